@@ -180,6 +180,25 @@ int64_t pxl_scaled_sum_work_bytes(void);
 int pxl_scaled_sum_noalloc(const float* v, int64_t n, double scale, float* out, void* stream);
 int64_t pxl_scaled_sum_noalloc_scratch_bytes(void);
 
+/* Bytes of the work buffer with which pxl_render_bwd_work / pxl_train_step_work scatter a
+ * trilinear batch of n_rays through tile bins (one 32-byte record per sample, summed per 8x8x8
+ * tile in LDS) instead of float atomics per corner; at most 12 GiB (larger batches run in
+ * pieces).  0: bins would not pay (nearest lookup, few samples per tile; grid->occupancy counts
+ * as a sparse scene) -- use the plain calls.
+ * Negative: an error code. */
+int64_t pxl_scatter_work_bytes(const pxl_grid* grid, const pxl_march* march, int64_t n_rays);
+
+/* pxl_render_bwd / pxl_train_step with a device work buffer of pxl_scatter_work_bytes (any
+ * smaller size works in more pieces; NULL or too small for two rays: the plain calls).  Its
+ * contents need no initialisation and are scratch afterwards.  grad_grid is added to, as in the
+ * plain calls; only the summation order differs. */
+int pxl_render_bwd_work(const pxl_grid* grid, const pxl_march* march, const pxl_rays* rays,
+                        const float* grad_rgba, const float* aux, float* grad_grid, void* work,
+                        int64_t work_bytes, void* stream);
+int pxl_train_step_work(const pxl_grid* grid, const pxl_march* march, const pxl_rays* rays,
+                        const pxl_loss* loss, float* out_rgba, float* grad_grid, void* work,
+                        int64_t work_bytes, void* stream);
+
 /* pxl_train_step with the trilinear gradient accumulated into corner blocks instead of
  * grad_grid: blocks is (X*Y*Z, 16) f32 (pxl_blocks_floats), zero on entry: one 64-byte entry
  * per cell E = (x, y, z), whose slot s = 2bx + by (floats 4s + c) receives channel c of corner

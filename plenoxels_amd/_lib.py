@@ -71,6 +71,11 @@ SIGNATURES = {
     "pxl_render_bwd": (ctypes.c_int, [_GP, _MP, _RP, c_void_p, c_void_p, c_void_p, c_void_p]),
     "pxl_train_step": (ctypes.c_int, [_GP, _MP, _RP, ctypes.POINTER(Loss), c_void_p, c_void_p,
                                       c_void_p]),
+    "pxl_scatter_work_bytes": (ctypes.c_int64, [_GP, _MP, ctypes.c_int64]),
+    "pxl_render_bwd_work": (ctypes.c_int, [_GP, _MP, _RP, c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_int64,
+                                           c_void_p]),
+    "pxl_train_step_work": (ctypes.c_int, [_GP, _MP, _RP, ctypes.POINTER(Loss), c_void_p, c_void_p, c_void_p,
+                                           ctypes.c_int64, c_void_p]),
     "pxl_train_step_blocks": (ctypes.c_int, [_GP, _MP, _RP, ctypes.POINTER(Loss), c_void_p, c_void_p,
                                              c_void_p]),
     "pxl_blocks_floats": (ctypes.c_int64, [_GP]),

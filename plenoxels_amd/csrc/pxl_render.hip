@@ -24,6 +24,7 @@
 #include <string>
 
 #include "pxl.h"
+#include "pxl_bins.h"
 #include "pxl_device.h"
 #include "pxl_host.h"
 
@@ -152,12 +153,12 @@ __global__ __launch_bounds__(kBlock) void k_render_fwd(KParams P, float* __restr
 // One group of the reverse sweep: given the group's clipped values, transmittance and Qn
 // (the suffix value just behind the group), emit dL/dvalue per sample, scatter it, and
 // return in Qn the suffix value in front of the group.
-template <int INTERP, bool RUNS = false>
+template <int INTERP, bool RUNS, bool BIN>
 __device__ __forceinline__ void reverse_chunk(const KParams& P, const Ray& R, int lane, int k,
                                               bool keep, const float4& v, uint32_t clip,
                                               float Ti, const float4& g, float beta_scale,
                                               float4& Qn, float* grad, uint32_t* s_cell,
-                                              float4* s_val) {
+                                              float4* s_val, const Bins& B, BinCursor& cur) {
   const float a = keep ? v.w : 0.f;
   Affine4 f;
   f.a0 = a * v.x;
@@ -184,15 +185,17 @@ __device__ __forceinline__ void reverse_chunk(const KParams& P, const Ray& R, in
     gv.w = Ti * (g.x * (v.x - s0) + g.y * (v.y - s1) + g.z * (v.z - s2) + g.w * (1.f - s3));
     if (beta_scale != 0.f) gv.w += beta_scale * beta_dloss(v.w);
   }
-  scatter_chunk<INTERP, RUNS>(P, R, lane, k, keep, clip, gv, grad, s_cell, s_val);
+  if constexpr (BIN) emit_chunk(P, B, R, lane, k, keep, gv, cur);
+  else scatter_chunk<INTERP, RUNS>(P, R, lane, k, keep, clip, gv, grad, s_cell, s_val);
   Qn = make_float4(readlane(f.a0, 0), readlane(f.a1, 0), readlane(f.a2, 0), readlane(f.a3, 0));
 }
 
 // Per-wave LDS of the kernels that scatter: the kept-sample list and, once the list has been
-// read into registers, the gradient staging area of scatter_chunk.
-template <int INTERP, int LIST>
+// read into registers, the gradient staging area of scatter_chunk (none with BIN: records go
+// straight to memory).
+template <int INTERP, int LIST, bool BIN = false>
 struct WaveLds {
-  static constexpr int kItems = ScatterItems<INTERP>::kPerChunk;
+  static constexpr int kItems = BIN ? 0 : ScatterItems<INTERP>::kPerChunk;
   static constexpr int kStage = kItems * 20;
   static constexpr int kBytes = (LIST * 4 > kStage ? LIST * 4 : kStage);
   static __device__ __forceinline__ int* list(unsigned char* base) { return reinterpret_cast<int*>(base); }
@@ -209,11 +212,13 @@ struct WaveLds {
 // are found again (`list`, kWave ints of LDS, may alias the staging area), re-gathered, and
 // their gradients -- the loss gradient g through the compositing, plus the beta term's
 // per-sample derivative when beta_scale != 0 -- scattered into grad.
-template <int DT, int INTERP, bool RUNS>
+template <int DT, int INTERP, bool RUNS, bool BIN>
 __device__ __forceinline__ void reverse_sweep(const KParams& P, const Ray& R, int lane, int* list,
                                               const float* grp, int ng, int n_proc, const float4& g,
-                                              float beta_scale, float* grad, uint32_t* s_cell, float4* s_val) {
+                                              float beta_scale, float* grad, uint32_t* s_cell, float4* s_val,
+                                              const Bins& B, BinCursor& cur) {
   float4 Qn = make_float4(0.f, 0.f, 0.f, 0.f);
+  const uint32_t slot0 = cur.slot;
   for (int gi = ng - 1; gi >= 0; --gi) {
     const float T0 = grp[2 * gi];
     const int k0 = __float_as_int(grp[2 * gi + 1]);
@@ -236,27 +241,41 @@ __device__ __forceinline__ void reverse_sweep(const KParams& P, const Ray& R, in
     if (valid) eval_kept<DT, INTERP>(P, R, k, v, clip);
     const float incl = wave_prefix_mul(1.f - v.w);
     const float Ti = T0 * wave_shift_up(incl, 1.f);
-    reverse_chunk<INTERP, RUNS>(P, R, lane, k, valid, v, clip, Ti, g, beta_scale, Qn, grad, s_cell, s_val);
+    if constexpr (BIN) cur.slot = slot0 + (uint32_t)(gi * kWave);
+    reverse_chunk<INTERP, RUNS, BIN>(P, R, lane, k, valid, v, clip, Ti, g, beta_scale, Qn, grad, s_cell, s_val, B, cur);
   }
 }
 
-template <int DT, int INTERP>
+// The cursor of a wave whose first ray is `ray` (local index within the launch) in a region of
+// `rays` rays.
+__device__ __forceinline__ BinCursor bin_cursor(const KParams& P, const Bins& B, uint32_t ray, uint32_t rays) {
+  return BinCursor{ray * (uint32_t)P.n_samples, ray / rays * B.run_cap, 0u};
+}
+
+template <int DT, int INTERP, bool BIN>
 __global__ __launch_bounds__(kBlock) void k_render_bwd(KParams P, const float* __restrict__ grad_out,
                                                         const float* __restrict__ aux,
-                                                        float* __restrict__ grad) {
-  using L = WaveLds<INTERP, kWave>;
+                                                        float* __restrict__ grad, Bins B) {
+  using L = WaveLds<INTERP, kWave, BIN>;
   __shared__ __align__(16) unsigned char s_mem[kWavesPerBlock][L::kBytes];
   const int lane = threadIdx.x & 63;
   const int64_t ray = wave_ray(P);
   if (ray >= P.n_rays) return;
+  const uint32_t region = (uint32_t)(ray - P.ray_offset);
+  BinCursor cur{};
+  if constexpr (BIN) cur = bin_cursor(P, B, region, 1u);
   const float4 g = reinterpret_cast<const float4*>(grad_out)[ray];
-  if (g.x == 0.f && g.y == 0.f && g.z == 0.f && g.w == 0.f) return;
+  if (g.x == 0.f && g.y == 0.f && g.z == 0.f && g.w == 0.f) {
+    if (BIN && lane == 0) B.n_runs[region] = 0u;
+    return;
+  }
   unsigned char* mem = s_mem[threadIdx.x >> 6];
   Ray R;
   setup_ray(P, ray, R);
   const float* ax = aux + ray * P.aux_stride;
-  reverse_sweep<DT, INTERP, false>(P, R, lane, L::list(mem), ax + 2, __float_as_int(ax[1]), __float_as_int(ax[0]), g,
-                                   0.f, grad, L::cells(mem), L::vals(mem));
+  reverse_sweep<DT, INTERP, false, BIN>(P, R, lane, L::list(mem), ax + 2, __float_as_int(ax[1]),
+                                        __float_as_int(ax[0]), g, 0.f, grad, L::cells(mem), L::vals(mem), B, cur);
+  if (BIN && lane == 0) B.n_runs[region] = cur.n;
 }
 
 // Training step for S <= 64*NG: every kept sample's value stays in registers between the
@@ -278,11 +297,12 @@ struct LossParams {
 template <int NG>
 constexpr bool kRunFlush = NG > 4;
 
-template <int DT, int INTERP, int NG>
+template <int DT, int INTERP, int NG, bool BIN>
 __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP, const Ray& R,
                                           int64_t ray, const float4& tgt, const int* list, int nk,
                                           int lane, uint32_t* s_cell, float4* s_val,
-                                          float* __restrict__ out, float* __restrict__ grad) {
+                                          float* __restrict__ out, float* __restrict__ grad,
+                                          const Bins& B, BinCursor& cur) {
   const int S = P.n_samples;
   const int ng = (nk + 63) >> 6;
   float4 V[NG];
@@ -333,13 +353,15 @@ __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP
   const float gs = LP.grad_scale;
   const float4 gl = make_float4(gs * d0, gs * d1, gs * d2, gs * d3);
   float4 Qn = make_float4(0.f, 0.f, 0.f, 0.f);
+  const uint32_t slot0 = cur.slot;
 #pragma unroll
   for (int g = NG - 1; g >= 0; --g) {
     // a group with no processed sample is the identity map: Qn passes through unchanged
     if (g < ng && KEEP[g] != 0ull) {
       const bool keep = (KEEP[g] >> lane) & 1ull;
-      reverse_chunk<INTERP, kRunFlush<NG>>(P, R, lane, KI[g], keep, V[g], CL[g], TI[g], gl, LP.beta_scale, Qn,
-                            grad, s_cell, s_val);
+      if constexpr (BIN) cur.slot = slot0 + (uint32_t)(g * kWave);
+      reverse_chunk<INTERP, kRunFlush<NG>, BIN>(P, R, lane, KI[g], keep, V[g], CL[g], TI[g], gl, LP.beta_scale, Qn,
+                                                grad, s_cell, s_val, B, cur);
     }
   }
 }
@@ -401,13 +423,14 @@ __device__ __forceinline__ Ray select_ray(bool second, const Ray& a, const Ray& 
 
 // Rays ray0 (lanes 0-31, list0[0..n0)) and ray0 + 1 (lanes 32-63, list1[0..n1)), n0, n1 <= 32,
 // one group of each; the steps of train_ray with T = 1 and Qn = 0.
-template <int DT, int INTERP, int NG>
+template <int DT, int INTERP, int NG, bool BIN>
 __device__ __forceinline__ void train_half_pair(const KParams& P, const LossParams& LP,
                                                 const Ray& R0, const Ray& R1, int64_t ray0,
                                                 bool has1, const float4& tgt0, const float4& tgt1,
                                                 const int* list0, int n0, const int* list1, int n1,
                                                 int lane, uint32_t* s_cell, float4* s_val,
-                                                float* __restrict__ out, float* __restrict__ grad) {
+                                                float* __restrict__ out, float* __restrict__ grad,
+                                                const Bins& B, BinCursor& cur) {
   const bool hi = lane >= 32;
   const int h = lane & 31;
   const bool valid = h < (hi ? n1 : n0);
@@ -477,15 +500,16 @@ __device__ __forceinline__ void train_half_pair(const KParams& P, const LossPara
     gv.w = Ti * (gl.x * (V.x - s0) + gl.y * (V.y - s1) + gl.z * (V.z - s2) + gl.w * (1.f - s3));
     if (LP.beta_scale != 0.f) gv.w += LP.beta_scale * beta_dloss(V.w);
   }
-  scatter_chunk<INTERP, kRunFlush<NG>>(P, R, lane, k, proc, CL, gv, grad, s_cell, s_val);
+  if constexpr (BIN) emit_chunk(P, B, R, lane, k, proc, gv, cur);
+  else scatter_chunk<INTERP, kRunFlush<NG>>(P, R, lane, k, proc, CL, gv, grad, s_cell, s_val);
 }
 
-template <int DT, int INTERP, int NG>
+template <int DT, int INTERP, int NG, bool BIN>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 && DT != PXL_DTYPE_F16 ? 5 : 1))) void k_train_pair(KParams P, LossParams LP,
                                                         float* __restrict__ out,
-                                                        float* __restrict__ grad) {
+                                                        float* __restrict__ grad, Bins B) {
   // per wave: [ray 0's list, then the scatter staging area | ray 1's list]
-  using L = WaveLds<INTERP, kWave * NG>;
+  using L = WaveLds<INTERP, kWave * NG, BIN>;
   constexpr int kList1 = kWave * NG * 4;
   __shared__ __align__(16) unsigned char s_mem[kWavesPerBlock][L::kBytes + kList1];
   const int lane = threadIdx.x & 63;
@@ -518,15 +542,21 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 
     n1 += __popcll(km1);
   }
   wave_lds_sync();
+  const uint32_t first = (uint32_t)(ray0 - P.ray_offset);
+  BinCursor cur{};
+  if constexpr (BIN) cur = bin_cursor(P, B, first, 2u);
   if (n0 <= 32 && n1 <= 32) {
-    train_half_pair<DT, INTERP, NG>(P, LP, R0, R1, ray0, has1, tgt0, tgt1, list0, n0, list1, n1, lane,
-                                L::cells(mem), L::vals(mem), out, grad);
+    train_half_pair<DT, INTERP, NG, BIN>(P, LP, R0, R1, ray0, has1, tgt0, tgt1, list0, n0, list1, n1, lane,
+                                         L::cells(mem), L::vals(mem), out, grad, B, cur);
   } else {
-    train_ray<DT, INTERP, NG>(P, LP, R0, ray0, tgt0, list0, n0, lane, L::cells(mem), L::vals(mem), out, grad);
+    train_ray<DT, INTERP, NG, BIN>(P, LP, R0, ray0, tgt0, list0, n0, lane, L::cells(mem), L::vals(mem), out, grad, B,
+                                   cur);
+    if constexpr (BIN) cur.slot = (first + 1u) * (uint32_t)P.n_samples;
     if (has1)
-      train_ray<DT, INTERP, NG>(P, LP, R1, ray0 + 1, tgt1, list1, n1, lane, L::cells(mem), L::vals(mem), out,
-                                grad);
+      train_ray<DT, INTERP, NG, BIN>(P, LP, R1, ray0 + 1, tgt1, list1, n1, lane, L::cells(mem), L::vals(mem), out,
+                                     grad, B, cur);
   }
+  if (BIN && lane == 0) B.n_runs[first >> 1] = cur.n;
 }
 
 // Training step for more than 512 samples per ray (up to 64 * kLongGroups): one ray per
@@ -538,10 +568,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 
 // flushes such stages by runs.
 constexpr int kLongGroups = PXL_TRAIN_MAX_SAMPLES / kWave;
 
-template <int DT, int INTERP>
+template <int DT, int INTERP, bool BIN>
 __global__ __launch_bounds__(kBlock) void k_train_long(KParams P, LossParams LP, float* __restrict__ out,
-                                                        float* __restrict__ grad) {
-  using L = WaveLds<INTERP, 2 * kWave>;  // the forward's sample buffer, then the scatter staging
+                                                        float* __restrict__ grad, Bins B) {
+  using L = WaveLds<INTERP, 2 * kWave, BIN>;  // the forward's sample buffer, then the scatter staging
   __shared__ __align__(16) unsigned char s_mem[kWavesPerBlock][L::kBytes];
   __shared__ float s_grp[kWavesPerBlock][2 * kLongGroups];
   const int lane = threadIdx.x & 63;
@@ -565,8 +595,12 @@ __global__ __launch_bounds__(kBlock) void k_train_long(KParams P, LossParams LP,
   wave_lds_sync();  // lane 0's group records are read by every lane
   const float gs = LP.grad_scale;
   const float4 gl = make_float4(gs * d0, gs * d1, gs * d2, gs * d3);
-  reverse_sweep<DT, INTERP, true>(P, R, lane, L::list(mem), grp, ng, n_proc, gl, LP.beta_scale, grad,
-                                  L::cells(mem), L::vals(mem));
+  const uint32_t region = (uint32_t)(ray - P.ray_offset);
+  BinCursor cur{};
+  if constexpr (BIN) cur = bin_cursor(P, B, region, 1u);
+  reverse_sweep<DT, INTERP, true, BIN>(P, R, lane, L::list(mem), grp, ng, n_proc, gl, LP.beta_scale, grad,
+                                       L::cells(mem), L::vals(mem), B, cur);
+  if (BIN && lane == 0) B.n_runs[region] = cur.n;
 }
 
 __global__ void k_camera_rays(KParams P, float* __restrict__ o, float* __restrict__ d,
@@ -1007,6 +1041,22 @@ using pxl_host::stride_blocks;
 
 constexpr int64_t kMaxRaysPerLaunch = int64_t(1) << 26;  // at most 2^24 blocks per launch
 
+// Tile bins (pxl_scatter_work_bytes): where they pay, by placed samples.  Their cost grows with
+// the tiles that are reached (each flushes up to ~240 requests), the corner atomics' with the kept
+// samples.  render_rays' backward, direct vs bins, in us: without occupancy (two thirds of the
+// samples kept) 128^3 cells, 4096 tiles: 44/50 at 2^18 samples, 80/64 at 2^19, 553/213 at 2^22;
+// 256^3, 32768 tiles: 505/525 at 2^22, 983/814 at 2^23; 48^3: 53/49 at 2^18, 193/113 at 2^20.
+// With a 5% occupancy (the host sees only that there is one): 128^3: 40/40 at 2^21, 73/56 at
+// 2^22; 256^3: 131/137 at 2^23; 48^3: 43/46 at 2^20, 132/87 at 2^22.
+constexpr double kBinMinSamples = double(1 << 19), kBinTileSamples = 160.0;
+constexpr double kBinMinSamplesOcc = double(1 << 22), kBinTileSamplesOcc = 512.0;
+// Largest work buffer (a 512^3 training step of 2^19 rays x 512 samples asks for 11.1 GB; in
+// three pieces of a third its tile sums take 2.7 instead of 1.2 ms), and the workgroups of the
+// tile sums, which stride over the items, whose number only the device knows: enough of them for
+// the hardware to balance tiles of different sizes (1536 resident: 0.85 ms there, 8192: 0.82).
+constexpr int64_t kBinMaxBytes = int64_t(12) << 30;
+constexpr unsigned kBinWorkgroups = 16384;
+
 int check_march(const pxl_march* m) {
   if (!m) return fail(PXL_E_INVALID, "march descriptor is NULL");
   if (m->n_samples < 0 || m->n_samples > (1 << 24))
@@ -1097,6 +1147,20 @@ int for_ray_pieces(pxl::KParams P, int64_t rays_per_block, F&& fn, const char* w
   return PXL_OK;
 }
 
+#define PXL_DISPATCH_DT(DT, ...)                                                      \
+  do {                                                                               \
+    if ((DT) == PXL_DTYPE_F32) {                                                     \
+      constexpr int kDT = PXL_DTYPE_F32;                                             \
+      __VA_ARGS__;                                                                   \
+    } else if ((DT) == PXL_DTYPE_BF16) {                                             \
+      constexpr int kDT = PXL_DTYPE_BF16;                                            \
+      __VA_ARGS__;                                                                   \
+    } else {                                                                         \
+      constexpr int kDT = PXL_DTYPE_F16;                                             \
+      __VA_ARGS__;                                                                   \
+    }                                                                                \
+  } while (0)
+
 #define PXL_DISPATCH_DT_INTERP(DT, INTERP, BODY)                                     \
   do {                                                                               \
     if ((DT) == PXL_DTYPE_F32) {                                                     \
@@ -1158,8 +1222,133 @@ int pxl_render_fwd(const pxl_grid* grid, const pxl_march* march, const pxl_rays*
   return rc;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The tile-binned scatter of a launch over rays [off, off + n): the bins laid out in `work`.
+// Everything but the counters is written before it is read.
+struct BinPlan {
+  int64_t tiles, run_cap, per_ray;  // run_cap: runs per ray
+  int64_t item_runs;
+  int64_t fixed;                    // bytes that do not grow with the rays
+};
+
+constexpr int64_t kBinAlign = 256;
+int64_t align_up(int64_t n) { return (n + kBinAlign - 1) / kBinAlign * kBinAlign; }
+
+BinPlan bin_plan(const pxl_grid* grid, const pxl_march* march) {
+  BinPlan p;
+  const int64_t S = march->n_samples;
+  p.tiles = occupancy_words(grid->dims[0], grid->dims[1], grid->dims[2]) / 16;
+  p.run_cap = pxl::bin_ray_runs(grid->dims[0], grid->dims[1], grid->dims[2], S);
+  p.item_runs = pxl::bin_item_runs(p.tiles);
+  p.per_ray = S * 32 + p.run_cap * (int64_t)(sizeof(pxl::BinRun) + sizeof(uint2)) + 4 +
+              (p.run_cap + p.item_runs - 1) / p.item_runs * (int64_t)sizeof(pxl::BinItem);
+  p.fixed = align_up((4 + p.tiles) * 4) + align_up(p.tiles * 4) + align_up(p.tiles * (int64_t)sizeof(pxl::BinItem)) +
+            8 * kBinAlign;
+  return p;
+}
+
+// Rays (even) whose bins fit work_bytes; 0: none.
+int64_t bin_rays(const BinPlan& p, int64_t S, int64_t work_bytes) {
+  int64_t n = work_bytes > p.fixed ? (work_bytes - p.fixed) / p.per_ray : 0;
+  n = std::min(n, (int64_t(1) << 31) / std::max<int64_t>(S, 1));  // 32-bit slots
+  return n & ~int64_t(1);
+}
+
+pxl::Bins bin_layout(const BinPlan& p, int64_t S, int64_t n, int64_t rays_per_region, void* work) {
+  char* w = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(work) + kBinAlign - 1) & ~uintptr_t(kBinAlign - 1));
+  auto take = [&w](int64_t bytes) {
+    char* q = w;
+    w += align_up(bytes);
+    return q;
+  };
+  pxl::Bins B{};
+  B.ctr = reinterpret_cast<uint32_t*>(take((4 + p.tiles) * 4));
+  B.tile_count = B.ctr + 4;
+  B.tile_base = reinterpret_cast<uint32_t*>(take(p.tiles * 4));
+  B.items = reinterpret_cast<pxl::BinItem*>(
+      take((p.tiles + n * ((p.run_cap + p.item_runs - 1) / p.item_runs)) * (int64_t)sizeof(pxl::BinItem)));
+  B.rec = reinterpret_cast<float4*>(take(n * S * 32));
+  B.runs = reinterpret_cast<pxl::BinRun*>(take(n * p.run_cap * (int64_t)sizeof(pxl::BinRun)));
+  B.sorted = reinterpret_cast<uint2*>(take(n * p.run_cap * (int64_t)sizeof(uint2)));
+  B.n_runs = reinterpret_cast<uint32_t*>(take(n * 4));
+  B.n_tiles = (uint32_t)p.tiles;
+  B.run_cap = (uint32_t)(p.run_cap * rays_per_region);
+  B.item_runs = (uint32_t)p.item_runs;
+  return B;
+}
+
+// Launch `fn(P, blocks, bins)` over all rays in pieces whose bins fit the work buffer, each
+// followed by the sort and the tile sums into grad_grid.
+template <typename F>
+int for_bin_pieces(const pxl_grid* grid, const pxl_march* march, pxl::KParams P, int64_t rays_per_block,
+                          int64_t rays_per_region, void* work, int64_t work_bytes, float* grad_grid, hipStream_t s,
+                          F&& fn, const char* what) {
+  const BinPlan plan = bin_plan(grid, march);
+  const int64_t per = std::min(bin_rays(plan, march->n_samples, work_bytes), (P.n_rays + 1) & ~int64_t(1));
+  const pxl::Bins B = bin_layout(plan, march->n_samples, per, rays_per_region, work);
+  const int64_t total = P.n_rays;
+  const int64_t zero4 = (4 + plan.tiles + 3) / 4;  // the layout rounds this up to whole float4s
+  for (int64_t off = 0; off < total; off += per) {
+    const int64_t n = std::min(per, total - off);
+    P.ray_offset = off;
+    P.n_rays = off + n;
+    hipLaunchKernelGGL(pxl::k_fill, dim3((unsigned)std::min<int64_t>((zero4 + 255) / 256, 4096)), dim3(256), 0, s,
+                       reinterpret_cast<float4*>(B.ctr), zero4, 0.f);
+    fn(P, (unsigned)((n + rays_per_block - 1) / rays_per_block), B);
+    hipLaunchKernelGGL(pxl::k_bin_tiles, dim3((unsigned)((plan.tiles + 256 * pxl::kTilesPerThread - 1) /
+                                                          (256 * pxl::kTilesPerThread))),
+                       dim3(256), 0, s, B);
+    const uint32_t regions = (uint32_t)((n + rays_per_region - 1) / rays_per_region);
+    hipLaunchKernelGGL(pxl::k_bin_place, dim3((regions + 15u) / 16u), dim3(256), 0, s, B, regions);
+#define PXL_BIN_ACC(DTV)                                                                                     \
+  hipLaunchKernelGGL(pxl::k_bin_accumulate<DTV>, dim3(kBinWorkgroups), dim3(256), 0, s, B, grid->data,       \
+                     (uint32_t)P.X, (uint32_t)P.Y, (uint32_t)P.Z, P.occ_ty, P.occ_tz, grad_grid)
+    if (grid->dtype == PXL_DTYPE_F32) PXL_BIN_ACC(PXL_DTYPE_F32);
+    else if (grid->dtype == PXL_DTYPE_BF16) PXL_BIN_ACC(PXL_DTYPE_BF16);
+    else PXL_BIN_ACC(PXL_DTYPE_F16);
+#undef PXL_BIN_ACC
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(e, what);
+  }
+  return PXL_OK;
+}
+
+// Whether a work buffer is used: trilinear, room for at least one pair of rays.
+bool use_bins(const pxl_grid* grid, const pxl_march* march, const void* work, int64_t work_bytes) {
+  return work != nullptr && march->interp == PXL_INTERP_TRILINEAR &&
+         bin_rays(bin_plan(grid, march), march->n_samples, work_bytes) > 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t pxl_scatter_work_bytes(const pxl_grid* grid, const pxl_march* march, int64_t n_rays) {
+  int rc;
+  if ((rc = check_grid(grid)) || (rc = check_march(march))) return rc;
+  if (n_rays < 0) return fail(PXL_E_INVALID, "n_rays is negative");
+  if (march->interp != PXL_INTERP_TRILINEAR || march->n_samples == 0) return 0;
+  const BinPlan p = bin_plan(grid, march);
+  const double samples = (double)n_rays * march->n_samples;
+  const bool occ = grid->occupancy != nullptr;
+  if (samples < (occ ? kBinMinSamplesOcc : kBinMinSamples) ||
+      samples < p.tiles * (occ ? kBinTileSamplesOcc : kBinTileSamples))
+    return 0;
+  const int64_t most = std::max<int64_t>(2, (kBinMaxBytes - p.fixed) / p.per_ray) & ~int64_t(1);
+  return p.fixed + p.per_ray * std::min<int64_t>(most, (n_rays + 1) & ~int64_t(1));
+}
+
 int pxl_render_bwd(const pxl_grid* grid, const pxl_march* march, const pxl_rays* rays,
                    const float* grad_rgba, const float* aux, float* grad_grid, void* stream) {
+  return pxl_render_bwd_work(grid, march, rays, grad_rgba, aux, grad_grid, nullptr, 0, stream);
+}
+
+int pxl_render_bwd_work(const pxl_grid* grid, const pxl_march* march, const pxl_rays* rays,
+                        const float* grad_rgba, const float* aux, float* grad_grid, void* work, int64_t work_bytes,
+                        void* stream) {
   int rc;
   if ((rc = check_grid(grid)) || (rc = check_march(march)) || (rc = check_rays(rays, false))) return rc;
   if (rays->n_rays == 0) return PXL_OK;
@@ -1167,18 +1356,44 @@ int pxl_render_bwd(const pxl_grid* grid, const pxl_march* march, const pxl_rays*
   if (march->n_samples == 0) return PXL_OK;
   pxl::KParams P = make_params(grid, march, rays);
   hipStream_t s = (hipStream_t)stream;
+  if (use_bins(grid, march, work, work_bytes)) {
+    constexpr int kIN = PXL_INTERP_TRILINEAR;
+    return for_bin_pieces(grid, march, P, pxl::kWavesPerBlock, 1, work, work_bytes, grad_grid, s,
+                          [&](const pxl::KParams& Q, unsigned nb, const pxl::Bins& B) {
+      PXL_DISPATCH_DT(grid->dtype, hipLaunchKernelGGL((pxl::k_render_bwd<kDT, kIN, true>), dim3(nb), dim3(pxl::kBlock),
+                                                      0, s, Q, grad_rgba, aux, grad_grid, B));
+    }, "pxl_render_bwd_work");
+  }
   PXL_DISPATCH_DT_INTERP(grid->dtype, march->interp, {
     rc = for_ray_pieces(P, pxl::kWavesPerBlock, [&](const pxl::KParams& Q, unsigned nb) {
-      hipLaunchKernelGGL((pxl::k_render_bwd<kDT, kIN>), dim3(nb), dim3(pxl::kBlock), 0, s, Q,
-                         grad_rgba, aux, grad_grid);
+      hipLaunchKernelGGL((pxl::k_render_bwd<kDT, kIN, false>), dim3(nb), dim3(pxl::kBlock), 0, s, Q,
+                         grad_rgba, aux, grad_grid, pxl::Bins{});
     }, "pxl_render_bwd");
   });
   return rc;
 }
 
-static int train_step(const pxl_grid* grid, const pxl_march* march, const pxl_rays* rays,
-                      const pxl_loss* loss, float* out_rgba, float* grad_grid, bool blocks,
-                      void* stream) {
+}  // extern "C"
+
+namespace {
+
+// k_train_pair / k_train_long over one piece of rays.
+template <int DT, int INTERP, bool BIN>
+void launch_train(const pxl::KParams& Q, const pxl::LossParams& LP, unsigned nb, float* out, float* grad,
+                         const pxl::Bins& B, hipStream_t s) {
+  const int S = Q.n_samples;
+#define PXL_LAUNCH_TRAIN(K) hipLaunchKernelGGL((K), dim3(nb), dim3(pxl::kBlock), 0, s, Q, LP, out, grad, B)
+  if (S > 512) PXL_LAUNCH_TRAIN((pxl::k_train_long<DT, INTERP, BIN>));
+  else if (S <= 64) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 1, BIN>));
+  else if (S <= 128) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 2, BIN>));
+  else if (S <= 256) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 4, BIN>));
+  else PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 8, BIN>));
+#undef PXL_LAUNCH_TRAIN
+}
+
+int train_step(const pxl_grid* grid, const pxl_march* march, const pxl_rays* rays,
+                      const pxl_loss* loss, float* out_rgba, float* grad_grid, bool blocks, void* work,
+                      int64_t work_bytes, void* stream) {
   int rc;
   if (!loss) return fail(PXL_E_INVALID, "loss descriptor is NULL");
   if ((rc = check_grid(grid)) || (rc = check_march(march)) ||
@@ -1198,48 +1413,44 @@ static int train_step(const pxl_grid* grid, const pxl_march* march, const pxl_ra
   if (rays->n_rays == 0) return PXL_OK;
   pxl::KParams P = make_params(grid, march, rays);
   P.corner_blocks = blocks ? 1 : 0;
-  pxl::LossParams LP{loss->targets, loss->grad_scale, loss->beta_scale, loss->ray_sq_err,
-                     loss->ray_beta};
+  const pxl::LossParams LP{loss->targets, loss->grad_scale, loss->beta_scale, loss->ray_sq_err,
+                           loss->ray_beta};  // per-ray arrays are indexed by the global ray number
   hipStream_t s = (hipStream_t)stream;
-  const int S = march->n_samples;
-  if (S > 512) {  // one ray per wavefront, group state in LDS (k_train_long)
-    PXL_DISPATCH_DT_INTERP(grid->dtype, march->interp, {
-      rc = for_ray_pieces(P, pxl::kWavesPerBlock, [&](const pxl::KParams& Q, unsigned nb) {
-        hipLaunchKernelGGL((pxl::k_train_long<kDT, kIN>), dim3(nb), dim3(pxl::kBlock), 0, s, Q, LP, out_rgba,
-                           grad_grid);
-      }, blocks ? "pxl_train_step_blocks" : "pxl_train_step");
-    });
-    return rc;
+  const bool pairs = march->n_samples <= 512;  // two rays per wavefront, eight per block; else one
+  const int64_t per_block = pairs ? 2 * pxl::kWavesPerBlock : pxl::kWavesPerBlock;
+  if (march->n_samples > 0 && use_bins(grid, march, work, work_bytes)) {
+    constexpr int kIN = PXL_INTERP_TRILINEAR;
+    return for_bin_pieces(grid, march, P, per_block, pairs ? 2 : 1, work, work_bytes, grad_grid, s,
+                          [&](const pxl::KParams& Q, unsigned nb, const pxl::Bins& B) {
+      PXL_DISPATCH_DT(grid->dtype, (launch_train<kDT, kIN, true>(Q, LP, nb, out_rgba, grad_grid, B, s)));
+    }, "pxl_train_step_work");
   }
   PXL_DISPATCH_DT_INTERP(grid->dtype, march->interp, {
-    // two rays per wavefront (k_train_pair), eight per block
-    rc = for_ray_pieces(P, 2 * pxl::kWavesPerBlock, [&](const pxl::KParams& Q, unsigned nb) {
-      const pxl::LossParams LQ = LP;  // per-ray arrays are indexed by the global ray number
-      if (S <= 64)
-        hipLaunchKernelGGL((pxl::k_train_pair<kDT, kIN, 1>), dim3(nb), dim3(pxl::kBlock), 0, s, Q,
-                           LQ, out_rgba, grad_grid);
-      else if (S <= 128)
-        hipLaunchKernelGGL((pxl::k_train_pair<kDT, kIN, 2>), dim3(nb), dim3(pxl::kBlock), 0, s, Q,
-                           LQ, out_rgba, grad_grid);
-      else if (S <= 256)
-        hipLaunchKernelGGL((pxl::k_train_pair<kDT, kIN, 4>), dim3(nb), dim3(pxl::kBlock), 0, s, Q,
-                           LQ, out_rgba, grad_grid);
-      else
-        hipLaunchKernelGGL((pxl::k_train_pair<kDT, kIN, 8>), dim3(nb), dim3(pxl::kBlock), 0, s, Q,
-                           LQ, out_rgba, grad_grid);
+    rc = for_ray_pieces(P, per_block, [&](const pxl::KParams& Q, unsigned nb) {
+      launch_train<kDT, kIN, false>(Q, LP, nb, out_rgba, grad_grid, pxl::Bins{}, s);
     }, blocks ? "pxl_train_step_blocks" : "pxl_train_step");
   });
   return rc;
 }
 
+}  // namespace
+
+extern "C" {
+
 int pxl_train_step(const pxl_grid* grid, const pxl_march* march, const pxl_rays* rays,
                    const pxl_loss* loss, float* out_rgba, float* grad_grid, void* stream) {
-  return train_step(grid, march, rays, loss, out_rgba, grad_grid, false, stream);
+  return train_step(grid, march, rays, loss, out_rgba, grad_grid, false, nullptr, 0, stream);
+}
+
+int pxl_train_step_work(const pxl_grid* grid, const pxl_march* march, const pxl_rays* rays,
+                        const pxl_loss* loss, float* out_rgba, float* grad_grid, void* work, int64_t work_bytes,
+                        void* stream) {
+  return train_step(grid, march, rays, loss, out_rgba, grad_grid, false, work, work_bytes, stream);
 }
 
 int pxl_train_step_blocks(const pxl_grid* grid, const pxl_march* march, const pxl_rays* rays,
                           const pxl_loss* loss, float* out_rgba, float* blocks, void* stream) {
-  return train_step(grid, march, rays, loss, out_rgba, blocks, true, stream);
+  return train_step(grid, march, rays, loss, out_rgba, blocks, true, nullptr, 0, stream);
 }
 
 int64_t pxl_blocks_floats(const pxl_grid* grid) {

@@ -151,6 +151,23 @@ class CameraRays:
                 raise ValueError("imgs and c2w must cover the same cameras")
 
 
+def _scatter_work(g, m, n_rays, device):
+    """The tile-bin work buffer of a scatter (pxl_scatter_work_bytes), or None where float atomics
+    are used: bins that would not pay, or a device without room for them (a quarter of the full
+    size also does, in more pieces)."""
+    n = _lib.lib().pxl_scatter_work_bytes(ctypes.byref(g), ctypes.byref(m), n_rays)
+    if n < 0:
+        _lib.check(int(n))
+    if n == 0:
+        return None
+    for size in (n, n // 4):
+        try:
+            return torch.empty(size, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            pass
+    return None
+
+
 class _RenderFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, grid, origins, dirs, cfg, occupancy, render_copy):
@@ -182,9 +199,10 @@ class _RenderFn(torch.autograd.Function):
         g = _grid_struct(src, occupancy)
         m = ctx.cfg.to_struct()
         r = _rays_struct(origins, dirs)
-        _lib.check(L.pxl_render_bwd(ctypes.byref(g), ctypes.byref(m), ctypes.byref(r),
-                                    _lib.ptr(grad_out), _lib.ptr(aux), _lib.ptr(grad),
-                                    _lib.stream_handle(src.device)))
+        work = _scatter_work(g, m, r.n_rays, src.device)
+        _lib.check(L.pxl_render_bwd_work(ctypes.byref(g), ctypes.byref(m), ctypes.byref(r),
+                                         _lib.ptr(grad_out), _lib.ptr(aux), _lib.ptr(grad), _lib.ptr(work),
+                                         0 if work is None else work.numel(), _lib.stream_handle(src.device)))
         return grad, None, None, None, None, None
 
 
@@ -367,8 +385,10 @@ def train_step(grid, grad_grid, *, cfg, origins=None, dirs=None, camera=None, ta
     m = cfg.to_struct()
     stream = _lib.stream_handle(grid.device)
     if blocks is None:
-        _lib.check(L.pxl_train_step(ctypes.byref(g), ctypes.byref(m), ctypes.byref(r), ctypes.byref(loss),
-                                    _lib.ptr(out), _lib.ptr(grad_grid), stream))
+        work = _scatter_work(g, m, R, grid.device)
+        _lib.check(L.pxl_train_step_work(ctypes.byref(g), ctypes.byref(m), ctypes.byref(r), ctypes.byref(loss),
+                                         _lib.ptr(out), _lib.ptr(grad_grid), _lib.ptr(work),
+                                         0 if work is None else work.numel(), stream))
     else:
         _lib.check(L.pxl_train_step_blocks(ctypes.byref(g), ctypes.byref(m), ctypes.byref(r), ctypes.byref(loss),
                                            _lib.ptr(out), _lib.ptr(blocks), stream))

@@ -1,0 +1,147 @@
+"""GPU parity of the tile-binned trilinear scatter (pxl_train_step_work, pxl_render_bwd_work)
+against the direct one (float atomics per corner) and the plain chain's autograd.
+
+Both add the same products; only the order of the float32 sums differs, as for the corner blocks,
+so the bars are theirs: 1e-5 relative between the two scatters, 1e-4 to autograd.
+"""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import plain
+from plenoxels_amd import MarchConfig, _lib, occupancy_dilate, pack_occupancy
+from plenoxels_amd.render import _grid_struct, _rays_struct, render_rays
+from util import grad_close, say
+
+DEV = torch.device("cuda:0")
+BASE = 2.0 ** -12
+
+
+def _scene(dims, R, S, seed):
+    """Rays through a grid of `dims` cells whose samples step about 1.2 cells and cross its faces."""
+    g = torch.Generator().manual_seed(seed)
+    pd = 0.1
+    grid = torch.rand(*dims, 4, generator=g) * 1.2 - 0.1
+    grid[..., 3] = grid[..., 3] * 0.2
+    gmin = torch.tensor([-0.4, 0.3, 0.0])
+    lo, size = gmin, torch.tensor(dims, dtype=torch.float32) * pd
+    a = lo + (torch.rand(R, 3, generator=g) * 1.4 - 0.2) * size
+    b = lo + torch.rand(R, 3, generator=g) * size
+    d = torch.nn.functional.normalize(b - a, dim=1)
+    delta = 0.12
+    o = b - d * (delta * S / 2)
+    return grid, o.contiguous(), d.contiguous(), tuple(gmin.tolist()), pd, delta, torch.rand(R, 4, generator=g)
+
+
+def _train(grid, o, d, tgt, cfg, bits, work):
+    L = _lib.lib()
+    out, sq = torch.empty(o.shape[0], 4, device=DEV), torch.empty(o.shape[0], device=DEV)
+    bsum = torch.empty(o.shape[0], device=DEV)
+    # added to, not overwritten; every addition rounds to 2^-24 of the sum, so a small base costs
+    # less than 1e-9 over the tens of additions a cell sees (a base of 0.25 would cost 1e-7 each)
+    grad = torch.full(grid.shape, BASE, dtype=torch.float32, device=DEV)
+    loss = _lib.Loss(targets=tgt.data_ptr(), grad_scale=0.5, beta_scale=1e-4, ray_sq_err=sq.data_ptr(),
+                     ray_beta=bsum.data_ptr())
+    g, m, r = _grid_struct(grid, bits), cfg.to_struct(), _rays_struct(o, d)
+    _lib.check(L.pxl_train_step_work(ctypes.byref(g), ctypes.byref(m), ctypes.byref(r), ctypes.byref(loss),
+                                     _lib.ptr(out), _lib.ptr(grad), _lib.ptr(work), 0 if work is None else work.numel(),
+                                     _lib.stream_handle(DEV)))
+    return out, sq, bsum, (grad - BASE).cpu()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims,R,S,dtype,occupied,t_stop", [
+    ((8, 8, 8), 65, 64, torch.float32, False, 0.0),       # one tile and its wrapped halo
+    ((9, 17, 5), 130, 65, torch.float32, True, 0.0),      # partial tiles, two groups
+    ((33, 10, 70), 257, 128, torch.bfloat16, False, 1e-2),
+    ((24, 24, 24), 1001, 256, torch.float16, True, 0.0),
+    ((40, 31, 16), 511, 300, torch.float32, False, 1e-2),
+    ((20, 20, 20), 3, 1, torch.float32, False, 0.0),
+    ((2, 1, 2), 64, 130, torch.float32, False, 0.0),
+    ((24, 20, 28), 300, 513, torch.float32, True, 0.0),   # one ray per wavefront
+    ((16, 50, 16), 129, 1100, torch.bfloat16, False, 0.0),
+])
+def test_binned_train_step_equals_direct(dims, R, S, dtype, occupied, t_stop):
+    say("bins", dims, R, S, dtype, occupied, t_stop)
+    grid, o, d, gmin, pd, delta, tgt = _scene(dims, R, S, 3)
+    grid, o, d, tgt = grid.to(dtype).to(DEV), o.to(DEV), d.to(DEV), tgt.to(DEV)
+    bits = None
+    if occupied:
+        occ = torch.rand(dims, generator=torch.Generator().manual_seed(4)) < 0.3
+        bits = occupancy_dilate(pack_occupancy(occ.to(DEV)), dims)
+    cfg = MarchConfig(S, delta, gmin, pd, "trilinear", 0.0, t_stop)
+    direct = _train(grid, o, d, tgt, cfg, bits, None)
+    assert direct[3].abs().max() > 0
+    whole = torch.full((1 << 26,), 0xA5, dtype=torch.uint8, device=DEV)  # its contents do not matter
+    # one piece, and an offset buffer that holds a few dozen rays at a time
+    for work in (whole, whole[3: 3 + (1 << 20) + 40 * 64 * S]):
+        binned = _train(grid, o, d, tgt, cfg, bits, work)
+        for a, b in zip(binned[:3], direct[:3]):
+            assert torch.equal(a, b)
+        ok, info = grad_close(binned[3], direct[3], rel=1e-5)
+        say("  ", work.numel(), info)
+        assert ok, info
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,interp", [(96, "trilinear"), (700, "trilinear"), (96, "nearest")])
+def test_render_rays_backward_above_the_bin_threshold(S, interp):
+    """Large enough a batch that render_rays' backward takes the bins (trilinear), against the plain
+    chain's autograd; some rays with a zero upstream gradient."""
+    R = (1 << 20) // S + 3
+    say("render_rays backward", R, S, interp)
+    grid, o, d, gmin, pd, delta, tgt = _scene((30, 22, 41), R, S, 5)
+    up = torch.rand(R, 4, generator=torch.Generator().manual_seed(6)) - 0.5
+    up[::7] = 0
+    leaf = grid.to(DEV).requires_grad_(True)
+    out = render_rays(leaf, o.to(DEV), d.to(DEV), num_samples=S, delta_step=delta, grid_min=gmin, points_distance=pd,
+                      interp=interp)
+    out.backward(up.to(DEV))
+    ref = grid.double().requires_grad_(True)
+    for a in range(0, R, 4096):
+        w = plain.render(ref, o[a:a + 4096], d[a:a + 4096], num_samples=S, delta_step=delta,
+                         gmin=torch.tensor(gmin), points_distance=pd, interp=interp, div_mode="reciprocal")
+        (w * up[a:a + 4096].double()).sum().backward()
+    ok, info = grad_close(leaf.grad.cpu(), ref.grad)
+    say("  ", info)
+    assert ok, info
+
+
+@pytest.mark.gpu
+def test_binned_integer_coordinates():
+    """Samples at exact integer coordinates (ceil == floor) and on the last cell, whose ceil is itself."""
+    X, pd = 16, 0.25
+    g = torch.Generator().manual_seed(70)
+    grid = (torch.rand(X, X, X, 4, generator=g) * 0.3).to(DEV)
+    o = torch.zeros(64, 3)
+    o[:, 0] = -3 * pd
+    o[:, 1:] = torch.randint(0, X, (64, 2), generator=g).float() * pd
+    d = torch.zeros(64, 3)
+    d[:, 0] = 1.0
+    tgt = torch.rand(64, 4, generator=g).to(DEV)
+    cfg = MarchConfig(24, pd, (0.0, 0.0, 0.0), pd, "trilinear")
+    a = _train(grid, o.to(DEV), d.to(DEV), tgt, cfg, None, None)[3]
+    b = _train(grid, o.to(DEV), d.to(DEV), tgt, cfg, None, torch.empty(1 << 24, dtype=torch.uint8, device=DEV))[3]
+    ok, info = grad_close(b, a, rel=1e-6)
+    say("bins at integer coordinates", info)
+    assert ok, info
+
+
+def test_scatter_work_bytes_rule():
+    """No buffer for nearest lookup, small batches and grids with many more tiles than samples; at
+    most 12 GiB; errors as the other entry points report them."""
+    L = _lib.lib()
+    g = _lib.Grid(data=0x1000, channels=4, dtype=_lib.DTYPE_F32)
+    for a, n in enumerate((64, 64, 64)):
+        g.dims[a] = n
+    tri, near = (MarchConfig(128, 0.1, (0.0, 0.0, 0.0), 0.1, i).to_struct() for i in ("trilinear", "nearest"))
+    q = lambda m, n: L.pxl_scatter_work_bytes(ctypes.byref(g), ctypes.byref(m), n)  # noqa: E731
+    assert q(near, 1 << 20) == 0 and q(tri, 0) == 0 and q(tri, 100) == 0
+    assert 0 < q(tri, 1 << 14) < q(tri, 1 << 15) <= q(tri, 1 << 26) <= 12 << 30
+    assert q(tri, -1) == _lib.PXL_E_INVALID
+    g.occupancy = 0x1000
+    assert q(tri, 1 << 14) == 0 and q(tri, 1 << 15) > 0
+    g.dims[0] = 1 << 18
+    assert q(tri, 1 << 14) == 0
+    assert L.pxl_scatter_work_bytes(None, ctypes.byref(tri), 5) == _lib.PXL_E_INVALID

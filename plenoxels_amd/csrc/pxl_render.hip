@@ -291,13 +291,13 @@ struct LossParams {
 // The train step of one ray after classification: its kept samples (list[0..nk)) in groups of
 // 64, loss and its gradient, the reverse sweep and the scatter.  `list` may alias the staging
 // area (s_cell, s_val): it is read completely before the first scatter.
-// The run flush of scatter_chunk goes into the train kernels for more than 256 samples per ray
-// (three waves per SIMD, registers to spare): the kernels for up to 256 samples keep five
-// waves per SIMD only without it (with it they spill or lose a wave).
-template <int NG>
-constexpr bool kRunFlush = NG > 4;
-
-template <int DT, int INTERP, int NG, bool BIN>
+// RUN: the run flush of scatter_chunk (trilinear).  It costs registers: the kernels for up to 256
+// samples keep five waves per SIMD only without it, so they have it where there is no occupancy
+// -- dense grids, whose rays keep runs of samples in one cell (64^3, 32768 rays x 128 samples into
+// corner blocks: 330 -> 243 us) -- and not for sparse scenes, whose samples rarely share a cell
+// (sparse256 spills and takes the flush in none of its stages).  Above 256 samples per ray (three
+// waves per SIMD) it is always there.
+template <int DT, int INTERP, int NG, bool BIN, bool RUN>
 __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP, const Ray& R,
                                           int64_t ray, const float4& tgt, const int* list, int nk,
                                           int lane, uint32_t* s_cell, float4* s_val,
@@ -360,7 +360,7 @@ __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP
     if (g < ng && KEEP[g] != 0ull) {
       const bool keep = (KEEP[g] >> lane) & 1ull;
       if constexpr (BIN) cur.slot = slot0 + (uint32_t)(g * kWave);
-      reverse_chunk<INTERP, kRunFlush<NG>, BIN>(P, R, lane, KI[g], keep, V[g], CL[g], TI[g], gl, LP.beta_scale, Qn,
+      reverse_chunk<INTERP, RUN, BIN>(P, R, lane, KI[g], keep, V[g], CL[g], TI[g], gl, LP.beta_scale, Qn,
                                                 grad, s_cell, s_val, B, cur);
     }
   }
@@ -423,7 +423,7 @@ __device__ __forceinline__ Ray select_ray(bool second, const Ray& a, const Ray& 
 
 // Rays ray0 (lanes 0-31, list0[0..n0)) and ray0 + 1 (lanes 32-63, list1[0..n1)), n0, n1 <= 32,
 // one group of each; the steps of train_ray with T = 1 and Qn = 0.
-template <int DT, int INTERP, int NG, bool BIN>
+template <int DT, int INTERP, int NG, bool BIN, bool RUN>
 __device__ __forceinline__ void train_half_pair(const KParams& P, const LossParams& LP,
                                                 const Ray& R0, const Ray& R1, int64_t ray0,
                                                 bool has1, const float4& tgt0, const float4& tgt1,
@@ -501,11 +501,11 @@ __device__ __forceinline__ void train_half_pair(const KParams& P, const LossPara
     if (LP.beta_scale != 0.f) gv.w += LP.beta_scale * beta_dloss(V.w);
   }
   if constexpr (BIN) emit_chunk(P, B, R, lane, k, proc, gv, cur);
-  else scatter_chunk<INTERP, kRunFlush<NG>>(P, R, lane, k, proc, CL, gv, grad, s_cell, s_val);
+  else scatter_chunk<INTERP, RUN>(P, R, lane, k, proc, CL, gv, grad, s_cell, s_val);
 }
 
-template <int DT, int INTERP, int NG, bool BIN>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 && DT != PXL_DTYPE_F16 ? 5 : 1))) void k_train_pair(KParams P, LossParams LP,
+template <int DT, int INTERP, int NG, bool BIN, bool RUN>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 && DT != PXL_DTYPE_F16 && !RUN ? 5 : 1))) void k_train_pair(KParams P, LossParams LP,
                                                         float* __restrict__ out,
                                                         float* __restrict__ grad, Bins B) {
   // per wave: [ray 0's list, then the scatter staging area | ray 1's list]
@@ -546,14 +546,14 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 
   BinCursor cur{};
   if constexpr (BIN) cur = bin_cursor(P, B, first, 2u);
   if (n0 <= 32 && n1 <= 32) {
-    train_half_pair<DT, INTERP, NG, BIN>(P, LP, R0, R1, ray0, has1, tgt0, tgt1, list0, n0, list1, n1, lane,
+    train_half_pair<DT, INTERP, NG, BIN, RUN>(P, LP, R0, R1, ray0, has1, tgt0, tgt1, list0, n0, list1, n1, lane,
                                          L::cells(mem), L::vals(mem), out, grad, B, cur);
   } else {
-    train_ray<DT, INTERP, NG, BIN>(P, LP, R0, ray0, tgt0, list0, n0, lane, L::cells(mem), L::vals(mem), out, grad, B,
+    train_ray<DT, INTERP, NG, BIN, RUN>(P, LP, R0, ray0, tgt0, list0, n0, lane, L::cells(mem), L::vals(mem), out, grad, B,
                                    cur);
     if constexpr (BIN) cur.slot = (first + 1u) * (uint32_t)P.n_samples;
     if (has1)
-      train_ray<DT, INTERP, NG, BIN>(P, LP, R1, ray0 + 1, tgt1, list1, n1, lane, L::cells(mem), L::vals(mem), out,
+      train_ray<DT, INTERP, NG, BIN, RUN>(P, LP, R1, ray0 + 1, tgt1, list1, n1, lane, L::cells(mem), L::vals(mem), out,
                                      grad, B, cur);
   }
   if (BIN && lane == 0) B.n_runs[first >> 1] = cur.n;
@@ -1382,12 +1382,17 @@ template <int DT, int INTERP, bool BIN>
 void launch_train(const pxl::KParams& Q, const pxl::LossParams& LP, unsigned nb, float* out, float* grad,
                          const pxl::Bins& B, hipStream_t s) {
   const int S = Q.n_samples;
+  constexpr bool kRuns = INTERP == PXL_INTERP_TRILINEAR && !BIN;
+  const bool dense = kRuns && Q.occ == nullptr;
 #define PXL_LAUNCH_TRAIN(K) hipLaunchKernelGGL((K), dim3(nb), dim3(pxl::kBlock), 0, s, Q, LP, out, grad, B)
   if (S > 512) PXL_LAUNCH_TRAIN((pxl::k_train_long<DT, INTERP, BIN>));
-  else if (S <= 64) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 1, BIN>));
-  else if (S <= 128) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 2, BIN>));
-  else if (S <= 256) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 4, BIN>));
-  else PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 8, BIN>));
+  else if (S > 256) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 8, BIN, kRuns>));
+  else if (S <= 64 && dense) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 1, BIN, kRuns>));
+  else if (S <= 64) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 1, BIN, false>));
+  else if (S <= 128 && dense) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 2, BIN, kRuns>));
+  else if (S <= 128) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 2, BIN, false>));
+  else if (dense) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 4, BIN, kRuns>));
+  else PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 4, BIN, false>));
 #undef PXL_LAUNCH_TRAIN
 }
 

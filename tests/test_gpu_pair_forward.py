@@ -1,0 +1,51 @@
+"""The two-rays-per-wavefront forward (occupancy given, up to 512 samples per ray) against the
+one-ray kernel: the same bits, outputs and saved state, for every chunk count, odd batches, rays
+with at most and with more than 32 kept samples, and early termination.  Without occupancy the
+one-ray kernel runs, so an occupancy of ones compares the two."""
+import ctypes
+
+import pytest
+import torch
+
+from plenoxels_amd import MarchConfig, _lib, pack_occupancy
+from plenoxels_amd.render import _grid_struct, _rays_struct
+from test_gpu_bins import _scene
+from util import say
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _forward(grid, o, d, cfg, bits):
+    L = _lib.lib()
+    R, n = o.shape[0], int(L.pxl_aux_floats(cfg.num_samples))
+    out, aux = torch.empty(R, 4, device=DEV), torch.zeros(R, n, device=DEV)
+    g, m, r = _grid_struct(grid, bits), cfg.to_struct(), _rays_struct(o, d)
+    for a in (aux, None):
+        _lib.check(L.pxl_render_fwd(ctypes.byref(g), ctypes.byref(m), ctypes.byref(r), _lib.ptr(out), _lib.ptr(a),
+                                    _lib.stream_handle(DEV)))
+        if a is not None:
+            first = out.clone()
+    assert torch.equal(first, out)
+    # only the groups that were walked are defined
+    ng = aux[:, 1].contiguous().view(torch.int32)
+    used = torch.arange(n, device=DEV)[None, :] < 2 + 2 * ng[:, None]
+    return out, torch.where(used, aux, torch.zeros_like(aux)).view(torch.int32)
+
+
+@pytest.mark.parametrize("S", [1, 64, 65, 128, 129, 256, 257, 512])
+@pytest.mark.parametrize("interp,t_stop,dtype", [("nearest", 0.0, torch.float32), ("trilinear", 0.05, torch.float32),
+                                                 ("trilinear", 0.0, torch.float16), ("nearest", 0.05, torch.bfloat16)])
+@pytest.mark.parametrize("dims", [(20, 20, 20), (70, 33, 40)])  # ~17 and ~40 samples per ray inside
+def test_pair_forward_equals_one_ray_forward(S, interp, t_stop, dtype, dims):
+    say("pair forward", S, interp, t_stop, dtype, dims)
+    R = 131
+    grid, o, d, gmin, pd, delta, _ = _scene(dims, R, S, 7)
+    grid = grid.to(dtype).to(DEV)
+    o[-1], d[-1] = o[0] + 100.0, d[0]  # a ray that misses
+    ones = pack_occupancy(torch.ones(dims, dtype=torch.bool, device=DEV))
+    cfg = MarchConfig(S, delta, gmin, pd, interp, 0.0, t_stop)
+    for n in (R, R - 1, 1):
+        a, ax = _forward(grid, o[:n].contiguous().to(DEV), d[:n].contiguous().to(DEV), cfg, None)
+        b, bx = _forward(grid, o[:n].contiguous().to(DEV), d[:n].contiguous().to(DEV), cfg, ones)
+        assert torch.equal(a, b) and torch.equal(ax, bx)

@@ -265,6 +265,10 @@ int pxl_occupancy_dilate(const uint32_t* occ_in, int64_t X, int64_t Y, int64_t Z
  * grid->occupancy is not read. */
 int pxl_alpha_occupancy(const pxl_grid* grid, int32_t dilate, uint32_t* bits, void* stream);
 
+/* pxl_alpha_occupancy and pxl_tv_sumsq of a float32 grid in one read of it. */
+int pxl_alpha_occupancy_tv(const pxl_grid* grid, int32_t dilate, uint32_t* bits, double* sum_sq,
+                           void* stream);
+
 /* Pack a (X,Y,Z) occupancy grid of bytes (nonzero = occupied) into the tile layout of
  * pxl_grid.occupancy.  out: pxl_occupancy_words(X, Y, Z) words (padding bits 0). */
 int pxl_pack_occupancy(const uint8_t* occ, int64_t X, int64_t Y, int64_t Z, uint32_t* out,

@@ -93,6 +93,7 @@ SIGNATURES = {
                                           c_void_p, c_void_p]),
     "pxl_occupancy_words": (ctypes.c_int64, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]),
     "pxl_alpha_occupancy": (ctypes.c_int, [_GP, ctypes.c_int32, c_void_p, c_void_p]),
+    "pxl_alpha_occupancy_tv": (ctypes.c_int, [_GP, ctypes.c_int32, c_void_p, c_void_p, c_void_p]),
     "pxl_fill_f32": (ctypes.c_int, [c_void_p, ctypes.c_int64, ctypes.c_float, c_void_p]),
     "pxl_fill_reachable_f32": (ctypes.c_int, [_GP, ctypes.c_int32, c_void_p, ctypes.c_float, c_void_p]),
     "pxl_sample_points": (ctypes.c_int, [c_void_p, ctypes.c_int64, c_void_p, ctypes.c_int64,

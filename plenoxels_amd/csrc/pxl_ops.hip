@@ -13,6 +13,7 @@
 
 #include "pxl.h"
 #include "pxl_device.h"
+#include "pxl_field.h"
 #include "pxl_host.h"
 
 using pxl_host::fail;
@@ -463,12 +464,7 @@ __global__ __launch_bounds__(256) void k_box_mean_adjoint(const float4* __restri
 
 // ---------------------------------------------------------------- total variation
 
-__device__ __forceinline__ double sq4(const float4& a, const float4& b) {
-  const float dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z, dw = a.w - b.w;
-  return (double)(dx * dx) + (double)(dy * dy) + (double)(dz * dz) + (double)(dw * dw);
-}
-
-// The TV kernels walk x columns: a workgroup covers 4 y rows (one wave each) x 64 z (the lanes)
+// The TV gradient kernels walk x columns: a workgroup covers 4 y rows (one wave each) x 64 z (the lanes)
 // and a slab of kTvSlab x planes, keeping each lane's x - 1, x and x + 1 cells in registers, so
 // the x neighbours (Y*Z cells apart, rarely still in cache when read in linear order) are read
 // once; the y and z neighbours are the lines the neighbouring waves and lanes load.
@@ -497,27 +493,6 @@ __device__ __forceinline__ TvUnit tv_unit(Dims d) {
 
 __host__ __device__ inline int64_t tv_units(int64_t X, int64_t Y, int64_t Z) {
   return ((X + kTvSlab - 1) / kTvSlab) * ((Y + 3) / 4) * ((Z + 63) / 64);
-}
-
-// sum over cells of the squared differences to the +y, +z and +x neighbours, in that order
-__global__ __launch_bounds__(256) void k_tv_sumsq(const float4* __restrict__ g, Dims d,
-                                                  double* __restrict__ sum) {
-  const uint32_t Y = (uint32_t)d.Y, Z = (uint32_t)d.Z, X = (uint32_t)d.X, YZ = Y * Z;
-  const TvUnit t = tv_unit(d);
-  double acc = 0.0;
-  if (t.active) {
-    float4 v = g[(int64_t)t.x0 * YZ + t.col];
-    for (uint32_t x = t.x0; x < t.x1; ++x) {
-      const int64_t L = (int64_t)x * YZ + t.col;
-      const float4 vx = x + 1 < X ? g[L + YZ] : make_float4(0.f, 0.f, 0.f, 0.f);
-      if (t.y + 1 < Y) acc += sq4(v, g[L + Z]);
-      if (t.z + 1 < Z) acc += sq4(v, g[L + 1]);
-      if (x + 1 < X) acc += sq4(v, vx);
-      v = vx;
-    }
-  }
-  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-  if ((threadIdx.x & 63) == 0) unsafeAtomicAdd(sum, acc);
 }
 
 // v - neighbour summed over +y, -y, +z, -z, +x, -x (in that order) for the cells of a column
@@ -1112,13 +1087,63 @@ int pxl_scaled_sum_noalloc(const float* v, int64_t n, double scale, float* out, 
   return launched("pxl_scaled_sum_noalloc");
 }
 
+}  // extern "C"
+
+namespace {
+
+template <int DT, bool OCC, bool TV>
+void launch_field(const void* grid, int64_t X, int64_t Y, int64_t Z, bool dilate, uint32_t* bits, double* sum,
+                  hipStream_t s) {
+  const uint32_t slab = pxl::field_slab(X, Y, Z);
+  const int64_t units = ((OCC ? (X + 7) / 8 * 8 : X) + slab - 1) / slab * ((Y + 7) / 8 * 2) * ((Z + 63) / 64);
+  const dim3 nb((unsigned)std::min<int64_t>(units, pxl::kFieldWorkgroups)), nt(pxl::kFieldThreads);
+  if (dilate)
+    hipLaunchKernelGGL((pxl::k_field<DT, true, OCC, TV>), nb, nt, 0, s, grid, (uint32_t)X, (uint32_t)Y, (uint32_t)Z,
+                       slab, bits, sum);
+  else
+    hipLaunchKernelGGL((pxl::k_field<DT, false, OCC, TV>), nb, nt, 0, s, grid, (uint32_t)X, (uint32_t)Y, (uint32_t)Z,
+                       slab, bits, sum);
+}
+
+int check_occupancy_out(const pxl_grid* grid, const uint32_t* bits) {
+  int rc;
+  if ((rc = pxl_host::check_grid(grid))) return rc;
+  if (!bits) return fail(PXL_E_INVALID, "bits is NULL");
+  return pxl_host::check_occupancy_words(grid->dims[0], grid->dims[1], grid->dims[2]);
+}
+
+}  // namespace
+
+extern "C" {
+
+int pxl_alpha_occupancy(const pxl_grid* grid, int32_t dilate, uint32_t* bits, void* stream) {
+  int rc;
+  if ((rc = check_occupancy_out(grid, bits))) return rc;
+  hipStream_t s = (hipStream_t)stream;
+  const int64_t *d = grid->dims;
+  if (grid->dtype == PXL_DTYPE_F32)
+    launch_field<PXL_DTYPE_F32, true, false>(grid->data, d[0], d[1], d[2], dilate != 0, bits, nullptr, s);
+  else if (grid->dtype == PXL_DTYPE_BF16)
+    launch_field<PXL_DTYPE_BF16, true, false>(grid->data, d[0], d[1], d[2], dilate != 0, bits, nullptr, s);
+  else
+    launch_field<PXL_DTYPE_F16, true, false>(grid->data, d[0], d[1], d[2], dilate != 0, bits, nullptr, s);
+  return launched("pxl_alpha_occupancy");
+}
+
+int pxl_alpha_occupancy_tv(const pxl_grid* grid, int32_t dilate, uint32_t* bits, double* sum_sq, void* stream) {
+  int rc;
+  if ((rc = check_occupancy_out(grid, bits)) || (rc = need(sum_sq != nullptr, "sum_sq is NULL"))) return rc;
+  if (grid->dtype != PXL_DTYPE_F32) return fail(PXL_E_DTYPE, "this entry point takes a float32 grid");
+  launch_field<PXL_DTYPE_F32, true, true>(grid->data, grid->dims[0], grid->dims[1], grid->dims[2], dilate != 0, bits,
+                                          sum_sq, (hipStream_t)stream);
+  return launched("pxl_alpha_occupancy_tv");
+}
+
 int pxl_tv_sumsq(const float* grid, int64_t X, int64_t Y, int64_t Z, double* sum_sq, void* stream) {
   int rc;
   if ((rc = pxl_host::check_dims(X, Y, Z)) || (rc = need(grid && sum_sq, "grid and sum_sq required")))
     return rc;
-  if (pxl::tv_units(X, Y, Z) > int64_t(0x7fffffff)) return fail(PXL_E_SIZE, "grid too large for pxl_tv_sumsq");
-  hipLaunchKernelGGL(pxl::k_tv_sumsq, dim3((unsigned)pxl::tv_units(X, Y, Z)), dim3(256), 0,
-                     (hipStream_t)stream, (const float4*)grid, Dims{X, Y, Z}, sum_sq);
+  launch_field<PXL_DTYPE_F32, false, true>(grid, X, Y, Z, false, nullptr, sum_sq, (hipStream_t)stream);
   return launched("pxl_tv_sumsq");
 }
 

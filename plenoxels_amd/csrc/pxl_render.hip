@@ -756,79 +756,6 @@ __global__ void k_dilate(const uint32_t* __restrict__ in, uint32_t X, uint32_t Y
   out[w] = word;
 }
 
-// Occupancy from the grid's own alpha: bit of cell (i, j, k) set when raw alpha >= 0 there
-// (DILATE: at any of the corners (i+a, j+b, k+c), a,b,c in {0,1}, wrapped -- the cells a
-// trilinear sample with floor cell (i, j, k) reads).  A sample whose cells all have raw alpha
-// < 0 is exactly zero in the reference's chain: clamp gives alpha 0, so its colour weight and
-// colour gradients vanish, and the clamp's gradient mask is 0 for every alpha it read.  NaN
-// alpha counts as empty.
-// A workgroup covers a y quad (y = 4q .. 4q+3, one wave each) and 64 consecutive z (the lanes,
-// so each wave reads whole runs of cells), and walks a slab of kAlphaOccSlab x planes: with
-// DILATE, plane x's "some corner (x, y+b, z+c) has alpha >= 0" is carried from the previous
-// step, so each plane's cells are read once.  Each wave's ballot holds one byte-row (y & 3) of
-// the 8 tile words along z; eight lanes assemble the words from the four ballots in LDS.
-// Units cover the padded dims (multiples of 8), so every word, padding included, is written.
-constexpr int kAlphaOccThreads = 256;
-constexpr uint32_t kAlphaOccSlab = 32;  // a multiple of 8: slabs cover whole tiles along x
-
-template <int DT, bool DILATE>
-__global__ __launch_bounds__(kAlphaOccThreads) void k_alpha_occupancy(const void* __restrict__ grid, uint32_t X,
-                                                                      uint32_t Y, uint32_t Z,
-                                                                      uint32_t* __restrict__ out) {
-  __shared__ uint64_t s_m[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint32_t TX = (X + 7u) >> 3, TY = (Y + 7u) >> 3, TZ = (Z + 7u) >> 3;
-  const uint32_t ZB = (TZ + 7u) >> 3, YQ = TY * 2u, XS = (TX * 8u + kAlphaOccSlab - 1u) / kAlphaOccSlab;
-  const uint64_t n_units = (uint64_t)XS * YQ * ZB;
-  for (uint64_t u = blockIdx.x; u < n_units; u += gridDim.x) {
-    const uint32_t zb = (uint32_t)(u % ZB), yq = (uint32_t)((u / ZB) % YQ), xs = (uint32_t)(u / ((uint64_t)ZB * YQ));
-    const uint32_t j = yq * 4u + (uint32_t)wave, k = zb * 64u + (uint32_t)lane;
-    const bool cell_ok = j < Y && k < Z;
-    const uint32_t j1 = j + 1 == Y ? 0u : j + 1, k1 = k + 1 == Z ? 0u : k + 1;
-    // any alpha >= 0 among plane i's corners (i, j+b, k+c) (DILATE) or at (i, j, k)
-    auto plane_any = [&](uint32_t i) {
-      if constexpr (DILATE) {
-        const uint32_t js[2] = {j, j1}, ks[2] = {k, k1};
-        bool any = false;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) any |= load_cell<DT>(grid, (i * Y + js[c >> 1]) * Z + ks[c & 1]).w >= 0.f;
-        return any;
-      } else {
-        return load_cell<DT>(grid, (i * Y + j) * Z + k).w >= 0.f;
-      }
-    };
-    const uint32_t x0 = xs * kAlphaOccSlab, x1 = min(TX * 8u, x0 + kAlphaOccSlab);
-    bool cur = DILATE && cell_ok && x0 < X ? plane_any(x0) : false;
-    for (uint32_t i = x0; i < x1; ++i) {
-      bool occ = false;
-      if (cell_ok && i < X) {
-        if constexpr (DILATE) {
-          const uint32_t i1 = i + 1 == X ? 0u : i + 1;
-          const bool nxt = plane_any(i1);
-          occ = cur | nxt;
-          cur = nxt;
-        } else {
-          occ = plane_any(i);
-        }
-      }
-      const uint64_t m = __ballot(occ);
-      if (lane == 0) s_m[wave] = m;
-      __syncthreads();
-      if (threadIdx.x < 8u) {  // tile word of z tile 8 zb + t
-        const uint32_t t = threadIdx.x, tz = zb * 8u + t;
-        if (tz < TZ) {
-          uint32_t word = 0u;
-#pragma unroll
-          for (int w = 0; w < 4; ++w) word |= (uint32_t)((s_m[w] >> (8u * t)) & 0xffu) << (8 * w);
-          const uint32_t tile = ((i >> 3) * TY + (yq >> 1)) * TZ + tz;
-          out[(size_t)tile * 16u + (i & 7u) * 2u + (yq & 1u)] = word;
-        }
-      }
-      __syncthreads();
-    }
-  }
-}
-
 // Bytes (X,Y,Z), nonzero = occupied, to occupancy tiles: one thread per output word.
 __global__ void k_pack_occupancy(const uint8_t* __restrict__ occ, uint32_t X, uint32_t Y, uint32_t Z,
                                  uint32_t* __restrict__ out, int64_t n_words) {
@@ -1671,34 +1598,6 @@ int pxl_occupancy_dilate(const uint32_t* occ_in, int64_t X, int64_t Y, int64_t Z
                      (hipStream_t)stream, occ_in, (uint32_t)X, (uint32_t)Y, (uint32_t)Z, occ_out, words);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? PXL_OK : hip_fail(e, "pxl_occupancy_dilate");
-}
-
-int pxl_alpha_occupancy(const pxl_grid* grid, int32_t dilate, uint32_t* bits, void* stream) {
-  int rc;
-  if ((rc = check_grid(grid))) return rc;
-  if (!bits) return fail(PXL_E_INVALID, "bits is NULL");
-  if ((rc = check_occupancy_words(grid->dims[0], grid->dims[1], grid->dims[2]))) return rc;
-  const int64_t units = (((grid->dims[0] + 7) / 8 * 8 + pxl::kAlphaOccSlab - 1) / pxl::kAlphaOccSlab) *
-                        ((grid->dims[1] + 7) / 8 * 2) * (((grid->dims[2] + 7) / 8 + 7) / 8);
-  const unsigned nb = (unsigned)std::min<int64_t>(units, int64_t(1) << 20);  // workgroup per unit
-  hipStream_t s = (hipStream_t)stream;
-  const uint32_t X = (uint32_t)grid->dims[0], Y = (uint32_t)grid->dims[1], Z = (uint32_t)grid->dims[2];
-#define PXL_ALPHA_OCC(DTV)                                                                           \
-  if (dilate)                                                                                        \
-    hipLaunchKernelGGL((pxl::k_alpha_occupancy<DTV, true>), dim3(nb), dim3(pxl::kAlphaOccThreads), 0, s,     \
-                       grid->data, X, Y, Z, bits);                                                   \
-  else                                                                                               \
-    hipLaunchKernelGGL((pxl::k_alpha_occupancy<DTV, false>), dim3(nb), dim3(pxl::kAlphaOccThreads), 0, s,    \
-                       grid->data, X, Y, Z, bits);
-  if (grid->dtype == PXL_DTYPE_F32) {
-    PXL_ALPHA_OCC(PXL_DTYPE_F32)
-  } else if (grid->dtype == PXL_DTYPE_BF16) {
-    PXL_ALPHA_OCC(PXL_DTYPE_BF16)
-  } else {
-    PXL_ALPHA_OCC(PXL_DTYPE_F16)
-  }
-#undef PXL_ALPHA_OCC
-  return launched("pxl_alpha_occupancy");
 }
 
 int pxl_pack_occupancy(const uint8_t* occ, int64_t X, int64_t Y, int64_t Z, uint32_t* out, void* stream) {

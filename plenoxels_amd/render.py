@@ -479,16 +479,20 @@ def occupancy_dilate(occ_bits, dims):
     return out
 
 
-def alpha_occupancy(grid, interp="nearest"):
+def alpha_occupancy(grid, interp="nearest", tv_sumsq=None):
     """Occupancy bits of the cells whose raw alpha is >= 0 (trilinear: floor cells any of whose
     8 corners is), from the grid itself (pxl_alpha_occupancy).  Skipping the other samples
     changes no finite result of the render and training kernels: their clamped alpha is 0 and
-    the clamp's gradient mask is 0."""
+    the clamp's gradient mask is 0.  tv_sumsq (float32 grids): a float64 device scalar to which
+    the same read of the grid adds optim.tv_sumsq's sum."""
     X, Y, Z = (int(v) for v in grid.shape[:3])
     bits = torch.empty(occupancy_words((X, Y, Z)), dtype=torch.int32, device=grid.device)
     g = _grid_struct(grid, None)
-    _lib.check(_lib.lib().pxl_alpha_occupancy(ctypes.byref(g), 1 if interp == "trilinear" else 0, _lib.ptr(bits),
-                                              _lib.stream_handle(grid.device)))
+    L, dilate, s = _lib.lib(), 1 if interp == "trilinear" else 0, _lib.stream_handle(grid.device)
+    if tv_sumsq is None:
+        _lib.check(L.pxl_alpha_occupancy(ctypes.byref(g), dilate, _lib.ptr(bits), s))
+    else:
+        _lib.check(L.pxl_alpha_occupancy_tv(ctypes.byref(g), dilate, _lib.ptr(bits), _lib.ptr(tv_sumsq), s))
     return bits
 
 

@@ -181,7 +181,13 @@ class Trainer:
             if key not in self._blocks:
                 self._blocks[key] = CornerBlockPair(grid)
             pair = self._blocks[key]
-        occ = alpha_occupancy(grid, self.interp) if self.skip_empty else None
+        use_tv = self.tv > 0 and k < 19
+        tv_grid = grid if grid.dtype == torch.float32 else self.grid
+        if use_tv:
+            self.tvs.zero_()
+        # the TV sum comes from the occupancy's read of the grid where both read the same one
+        tv_with_occ = use_tv and self.skip_empty and tv_grid is grid
+        occ = alpha_occupancy(grid, self.interp, self.tvs if tv_with_occ else None) if self.skip_empty else None
         if pooled_blocks:
             key = tuple(grid.shape[:3])
             if self._pooled_pair is None or self._pooled_pair[0] != key:
@@ -203,11 +209,10 @@ class Trainer:
         loss = closs
         # full-grid steps with the TV term fold its backward into the Adam pass (pxl_adam_tv_step,
         # the same bits), which writes the updated grid into a second buffer
-        fused_tv = self.tv > 0 and k < 19 and not pooled
-        if self.tv > 0 and k < 19:
-            tv_grid = grid if grid.dtype == torch.float32 else self.grid
-            self.tvs.zero_()
-            tv_sumsq(tv_grid, out=self.tvs)
+        fused_tv = use_tv and not pooled
+        if use_tv:
+            if not tv_with_occ:
+                tv_sumsq(tv_grid, out=self.tvs)
             if not fused_tv:
                 tv_backward_(tv_grid, self.tvs, self.tv, grad)
             tvl = (self.tv * torch.sqrt(self.tvs)).float().reshape(())

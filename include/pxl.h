@@ -378,6 +378,9 @@ int pxl_tv_sumsq(const float* grid, int64_t X, int64_t Y, int64_t Z, double* sum
 /* d(weight * sqrt(sum_sq))/dgrid accumulated into grad_grid; sum_sq read on the device. */
 int pxl_tv_bwd(const float* grid, int64_t X, int64_t Y, int64_t Z, const double* sum_sq,
                float weight, float* grad_grid, void* stream);
+/* The same written to grad_grid (every cell), with the weight read on the device (one float). */
+int pxl_tv_grad(const float* grid, int64_t X, int64_t Y, int64_t Z, const double* sum_sq,
+                const float* weight, float* grad_grid, void* stream);
 
 /* torch.optim.Adam step (scripts/train.py:89,182; defaults betas (0.9,0.999), eps 1e-8, no
  * weight decay) fused with the |grad| accumulation of scripts/train.py:184:

@@ -131,6 +131,8 @@ SIGNATURES = {
                                     c_void_p]),
     "pxl_tv_bwd": (ctypes.c_int, [c_void_p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, c_void_p,
                                   ctypes.c_float, c_void_p, c_void_p]),
+    "pxl_tv_grad": (ctypes.c_int, [c_void_p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, c_void_p, c_void_p,
+                                   c_void_p, c_void_p]),
     "pxl_adam_step": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_int64,
                                      ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double,
                                      ctypes.c_int64, c_void_p, ctypes.c_int32, c_void_p]),

@@ -665,6 +665,18 @@ __device__ __forceinline__ int merge_nearest_runs(int lane, int ns, uint32_t* s_
   return __popcll(tails);
 }
 
+// Items 0 .. n-1 added to grad, four lanes per item: one memory request per cell.
+__device__ __forceinline__ void flush_cells(int lane, int n, float* grad, const uint32_t* s_cell, const float* sv) {
+  const int ch = lane & 3;
+  for (int base = 0; base < n; base += kWave / 4) {
+    const int it = base + (lane >> 2);
+    if (it < n) {
+      const float v = sv[4 * it + ch];
+      if (v != 0.f) atomic_add_f32(grad + (size_t)s_cell[it] * 4u + ch, v);
+    }
+  }
+}
+
 template <int INTERP, bool RUNS = false>
 __device__ __forceinline__ void scatter_chunk(const KParams& P, const Ray& R, int lane, int k,
                                               bool keep, uint32_t clip, const float4& gv,
@@ -703,15 +715,7 @@ __device__ __forceinline__ void scatter_chunk(const KParams& P, const Ray& R, in
         }
       }
     }
-    if (!by_runs) {
-      for (int base = 0; base < n; base += kWave / 4) {
-        const int it = base + (lane >> 2);
-        if (it < n) {
-          const float v = sv[4 * it + ch];
-          if (v != 0.f) atomic_add_f32(grad + (size_t)s_cell[it] * 4u + ch, v);
-        }
-      }
-    }
+    if (!by_runs) flush_cells(lane, n, grad, s_cell, sv);
     wave_lds_sync();
   }
 }

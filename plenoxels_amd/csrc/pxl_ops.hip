@@ -75,33 +75,66 @@ __global__ void k_init_min(float* out3) {
   if (threadIdx.x < 3) out3[threadIdx.x] = INFINITY;
 }
 
+// *a = min(*a, v) by integer order: floats of one sign order as their bits, negative ones in
+// reverse, and every negative float is below every positive one as a signed integer.
 __device__ __forceinline__ void atomic_min_f32(float* a, float v) {
-  unsigned int* ai = reinterpret_cast<unsigned int*>(a);
-  unsigned int old = *ai;
-  while (v < __uint_as_float(old)) {
-    const unsigned int prev = atomicCAS(ai, old, __float_as_uint(v));
-    if (prev == old) break;
-    old = prev;
-  }
+  const int bits = __float_as_int(v);
+  if (bits >= 0) atomicMin(reinterpret_cast<int*>(a), bits);
+  else atomicMax(reinterpret_cast<unsigned int*>(a), (unsigned int)bits);
 }
 
-__global__ void k_coord_min(const float* __restrict__ c, int64_t n, float* out3) {
-  float m0 = INFINITY, m1 = INFINITY, m2 = INFINITY;
-  PXL_GRID_STRIDE(i, n) {
-    m0 = fminf(m0, c[3 * i]);
-    m1 = fminf(m1, c[3 * i + 1]);
-    m2 = fminf(m2, c[3 * i + 2]);
+// Column minima of (n,3) read as float4s where the array is 16-byte aligned: float4 i starts at
+// column i mod 3, which stays the same for a thread whose stride is a multiple of 3 (the grid
+// is), so each thread keeps one minimum per component and rotates them at the end.  One atomic
+// per column and workgroup.  16.8 M points (a 256^3 grid's coordinates): 154 us with three strided
+// loads per point and a compare-and-swap loop per wave, 71 us so.
+constexpr int kMinBlocks = 3 * 512;
+
+__global__ __launch_bounds__(256) void k_coord_min(const float* __restrict__ c, int64_t n, int vec, float* out3) {
+  __shared__ float s_min[4][3];
+  float a[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
+  const int64_t tid = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
+  const int64_t n4 = vec ? n * 3 / 4 : 0;
+  const float4* c4 = reinterpret_cast<const float4*>(c);
+  int64_t i4 = tid;
+  for (; i4 + 3 * stride < n4; i4 += 4 * stride) {  // four loads in flight
+    const float4 p = c4[i4], q = c4[i4 + stride], r = c4[i4 + 2 * stride], t = c4[i4 + 3 * stride];
+    a[0] = fminf(a[0], fminf(fminf(p.x, q.x), fminf(r.x, t.x)));
+    a[1] = fminf(a[1], fminf(fminf(p.y, q.y), fminf(r.y, t.y)));
+    a[2] = fminf(a[2], fminf(fminf(p.z, q.z), fminf(r.z, t.z)));
+    a[3] = fminf(a[3], fminf(fminf(p.w, q.w), fminf(r.w, t.w)));
   }
-  for (int off = 32; off > 0; off >>= 1) {
-    m0 = fminf(m0, __shfl_xor(m0, off));
-    m1 = fminf(m1, __shfl_xor(m1, off));
-    m2 = fminf(m2, __shfl_xor(m2, off));
+  for (; i4 < n4; i4 += stride) {
+    const float4 v = c4[i4];
+    a[0] = fminf(a[0], v.x);
+    a[1] = fminf(a[1], v.y);
+    a[2] = fminf(a[2], v.z);
+    a[3] = fminf(a[3], v.w);
   }
-  if ((threadIdx.x & 63) == 0) {
-    atomic_min_f32(out3 + 0, m0);
-    atomic_min_f32(out3 + 1, m1);
-    atomic_min_f32(out3 + 2, m2);
+  float m[3];
+  const int phase = (int)(tid % 3);  // column of component 0 (and 3)
+#pragma unroll
+  for (int col = 0; col < 3; ++col) {
+    const int comp = (col - phase + 3) % 3;
+    m[col] = comp == 0 ? fminf(a[0], a[3]) : comp == 1 ? a[1] : a[2];
   }
+  for (int64_t i = 4 * n4 + tid; i < 3 * n; i += stride) {  // the rest, or everything unaligned
+    const int col = (int)(i % 3);
+    const float v = c[i];
+    m[0] = col == 0 ? fminf(m[0], v) : m[0];
+    m[1] = col == 1 ? fminf(m[1], v) : m[1];
+    m[2] = col == 2 ? fminf(m[2], v) : m[2];
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int col = 0; col < 3; ++col) {
+    for (int off = 32; off > 0; off >>= 1) m[col] = fminf(m[col], __shfl_xor(m[col], off));
+    if (lane == 0) s_min[wave][col] = m[col];
+  }
+  __syncthreads();
+  if (threadIdx.x < 3)
+    atomic_min_f32(out3 + threadIdx.x, fminf(fminf(s_min[0][threadIdx.x], s_min[1][threadIdx.x]),
+                                             fminf(s_min[2][threadIdx.x], s_min[3][threadIdx.x])));
 }
 
 __global__ void k_normalize(const float* __restrict__ p, int64_t n, const float* __restrict__ m3,
@@ -142,13 +175,24 @@ __global__ void k_wrap(int64_t* __restrict__ idx, int64_t n, Dims d) {
   }
 }
 
+// Wrapped index of a rounded coordinate: itself inside, a 32-bit remainder where it fits (dims are
+// below 2^31; a 64-bit remainder takes several times as long), else the 64-bit one.
+__device__ __forceinline__ uint32_t wrap_rounded(float r, int64_t dim) {
+  if (r >= 0.f && r < (float)dim) return (uint32_t)r;
+  if (fabsf(r) < 1.0e9f) {
+    const int m = (int)r % (int)dim;
+    return (uint32_t)(m < 0 ? m + (int)dim : m);
+  }
+  return (uint32_t)pymod(to_i64(r), dim);
+}
+
 // idx = round-half-even(n).long(); mask = in-bounds; cell = wrapped idx
-__device__ __forceinline__ int64_t nearest_wrapped(const float* n, int64_t i, const Dims& d,
-                                                   bool& inb) {
-  const int64_t a = to_i64(__builtin_rintf(n[3 * i])), b = to_i64(__builtin_rintf(n[3 * i + 1])),
-                c = to_i64(__builtin_rintf(n[3 * i + 2]));
+__device__ __forceinline__ uint32_t nearest_wrapped(const float* n, int64_t i, const Dims& d, bool& inb) {
+  const float x = __builtin_rintf(n[3 * i]), y = __builtin_rintf(n[3 * i + 1]), z = __builtin_rintf(n[3 * i + 2]);
+  const int64_t a = to_i64(x), b = to_i64(y), c = to_i64(z);
   inb = a >= 0 && a < d.X && b >= 0 && b < d.Y && c >= 0 && c < d.Z;
-  return cell_of(d, pymod(a, d.X), pymod(b, d.Y), pymod(c, d.Z));
+  if (inb) return (uint32_t)cell_of(d, a, b, c);
+  return (uint32_t)cell_of(d, wrap_rounded(x, d.X), wrap_rounded(y, d.Y), wrap_rounded(z, d.Z));
 }
 
 __global__ void k_nearest_gather(const float* __restrict__ n, int64_t N, Dims d,
@@ -156,18 +200,39 @@ __global__ void k_nearest_gather(const float* __restrict__ n, int64_t N, Dims d,
                                  uint8_t* __restrict__ mask) {
   PXL_GRID_STRIDE(i, N) {
     bool inb;
-    const int64_t cell = nearest_wrapped(n, i, d, inb);
+    const uint32_t cell = nearest_wrapped(n, i, d, inb);
     vals[i] = grid[cell];
     if (mask) mask[i] = inb;
   }
 }
 
-__global__ void k_nearest_scatter(const float* __restrict__ n, int64_t N, Dims d,
-                                  const float4* __restrict__ g, float* __restrict__ grad) {
-  PXL_GRID_STRIDE(i, N) {
-    bool inb;
-    const int64_t cell = nearest_wrapped(n, i, d, inb);
-    atomic_add4(grad + 4 * cell, g[i]);
+// Gradient rows into the grid, 64 points per wave: the nonzero rows are compacted in LDS (a caller
+// that masked its out-of-grid samples leaves them zero), runs of one cell merged where a quarter
+// of the points repeat the previous one's, and added four lanes per cell, so that a row is one
+// memory request and not one per channel.  7.3 M points of 600-sample rays: 180 us with an atomic
+// per point and channel, 137 us so.
+__global__ __launch_bounds__(256) void k_nearest_scatter(const float* __restrict__ n, int64_t N, Dims d,
+                                                         const float4* __restrict__ g, float* __restrict__ grad) {
+  __shared__ uint32_t s_cell[kWavesPerBlock][kWave];
+  __shared__ float4 s_val[kWavesPerBlock][kWave];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t base = (int64_t)blockIdx.x * blockDim.x + wave * kWave; base < N; base += stride) {
+    const int64_t i = base + lane;
+    const float4 v = i < N ? g[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const bool keep = v.x != 0.f || v.y != 0.f || v.z != 0.f || v.w != 0.f;
+    const uint64_t km = __ballot(keep);
+    if (km == 0ull) continue;
+    if (keep) {
+      bool inb;
+      const int r = lane_rank(km);
+      s_cell[wave][r] = nearest_wrapped(n, i, d, inb);
+      s_val[wave][r] = v;
+    }
+    wave_lds_sync();
+    flush_cells(lane, merge_nearest_runs(lane, __popcll(km), s_cell[wave], s_val[wave]), grad, s_cell[wave],
+                reinterpret_cast<const float*>(s_val[wave]));
+    wave_lds_sync();
   }
 }
 
@@ -468,7 +533,10 @@ __global__ __launch_bounds__(256) void k_box_mean_adjoint(const float4* __restri
 // and a slab of kTvSlab x planes, keeping each lane's x - 1, x and x + 1 cells in registers, so
 // the x neighbours (Y*Z cells apart, rarely still in cache when read in linear order) are read
 // once; the y and z neighbours are the lines the neighbouring waves and lanes load.
-constexpr int kTvSlab = 64;
+// The gradient kernel takes 32 planes where 64 would leave fewer than 2048 workgroups (256^3: 154
+// against 199 us); the Adam pass, whose nine other streams fill the memory system, does not (256^3:
+// 494 us with 64 planes, 620 with 32).
+constexpr uint32_t kTvSlab = 64;
 
 struct TvUnit {
   uint32_t x0, x1, y, z;
@@ -476,7 +544,7 @@ struct TvUnit {
   bool active;
 };
 
-__device__ __forceinline__ TvUnit tv_unit(Dims d) {
+__device__ __forceinline__ TvUnit tv_unit(Dims d, uint32_t slab) {
   const uint32_t Y = (uint32_t)d.Y, Z = (uint32_t)d.Z, X = (uint32_t)d.X;
   const uint32_t nzb = (Z + 63u) / 64u, nyb = (Y + 3u) / 4u;
   const uint32_t u = blockIdx.x;
@@ -484,15 +552,19 @@ __device__ __forceinline__ TvUnit tv_unit(Dims d) {
   TvUnit t;
   t.y = yb * 4u + (threadIdx.x >> 6);
   t.z = zb * 64u + (threadIdx.x & 63u);
-  t.x0 = xs * kTvSlab;
-  t.x1 = min(X, t.x0 + kTvSlab);
+  t.x0 = xs * slab;
+  t.x1 = min(X, t.x0 + slab);
   t.active = t.y < Y && t.z < Z && t.x0 < X;
   t.col = (int64_t)t.y * Z + t.z;
   return t;
 }
 
-__host__ __device__ inline int64_t tv_units(int64_t X, int64_t Y, int64_t Z) {
-  return ((X + kTvSlab - 1) / kTvSlab) * ((Y + 3) / 4) * ((Z + 63) / 64);
+inline int64_t tv_units(int64_t X, int64_t Y, int64_t Z, int64_t slab = kTvSlab) {
+  return ((X + slab - 1) / slab) * ((Y + 3) / 4) * ((Z + 63) / 64);
+}
+
+inline uint32_t tv_bwd_slab(int64_t X, int64_t Y, int64_t Z) {
+  return tv_units(X, Y, Z) < 2048 ? kTvSlab / 2 : kTvSlab;
 }
 
 // v - neighbour summed over +y, -y, +z, -z, +x, -x (in that order) for the cells of a column
@@ -517,13 +589,18 @@ __device__ __forceinline__ float4 tv_dir(const float4* __restrict__ g, int64_t L
   return acc;
 }
 
-__global__ __launch_bounds__(256) void k_tv_bwd(const float4* __restrict__ g, Dims d,
+// d/dx of weight*sqrt(S): weight / sqrt(S) * sum over neighbours of (x - neighbour), added to grad
+// (weight from the host) or, with WRITE, grad itself (weight_dev: a device scalar, so that
+// autograd's upstream gradient needs no synchronisation).
+// 256^3: 233 us adding to a zeroed gradient (and 40 for the zeros), 154 written.
+template <bool WRITE>
+__global__ __launch_bounds__(256) void k_tv_bwd(const float4* __restrict__ g, Dims d, uint32_t slab,
                                                 const double* __restrict__ sum, float weight,
+                                                const float* __restrict__ weight_dev,
                                                 float4* __restrict__ grad) {
-  // d/dx of weight*sqrt(S): weight / sqrt(S) * sum over neighbours of (x - neighbour)
-  const float scale = weight / (float)sqrt(*sum);
+  const float scale = (WRITE ? *weight_dev : weight) / (float)sqrt(*sum);
   const uint32_t Y = (uint32_t)d.Y, Z = (uint32_t)d.Z, X = (uint32_t)d.X, YZ = Y * Z;
-  const TvUnit t = tv_unit(d);
+  const TvUnit t = tv_unit(d, slab);
   if (!t.active) return;
   float4 vm = t.x0 > 0 ? g[(int64_t)(t.x0 - 1) * YZ + t.col] : make_float4(0.f, 0.f, 0.f, 0.f);
   float4 v = g[(int64_t)t.x0 * YZ + t.col];
@@ -531,7 +608,7 @@ __global__ __launch_bounds__(256) void k_tv_bwd(const float4* __restrict__ g, Di
     const int64_t L = (int64_t)x * YZ + t.col;
     const float4 vp = x + 1 < X ? g[L + YZ] : make_float4(0.f, 0.f, 0.f, 0.f);
     const float4 acc = tv_dir(g, L, v, vm, vp, x, t.y, t.z, X, Y, Z, YZ);
-    float4 c = grad[L];
+    float4 c = WRITE ? make_float4(0.f, 0.f, 0.f, 0.f) : grad[L];
     c.x += scale * acc.x;
     c.y += scale * acc.y;
     c.z += scale * acc.z;
@@ -633,7 +710,7 @@ __global__ __launch_bounds__(256) void k_adam_tv(const float4* __restrict__ p_in
                                                  int zero_grad) {
   const float scale = weight / (float)sqrt(*sum);
   const uint32_t Y = (uint32_t)d.Y, Z = (uint32_t)d.Z, X = (uint32_t)d.X, YZ = Y * Z;
-  const TvUnit t = tv_unit(d);
+  const TvUnit t = tv_unit(d, kTvSlab);
   if (!t.active) return;  // no cross-lane operations below
   float4 Pm = t.x0 > 0 ? p_in[(int64_t)(t.x0 - 1) * YZ + t.col] : make_float4(0.f, 0.f, 0.f, 0.f);
   float4 P = p_in[(int64_t)t.x0 * YZ + t.col];
@@ -833,8 +910,9 @@ int pxl_coord_min(const float* coords, int64_t n, float* out3, void* stream) {
   int rc;
   if ((rc = need(coords && out3 && n > 0, "coords, out3 and n > 0 are required"))) return rc;
   hipLaunchKernelGGL(pxl::k_init_min, dim3(1), dim3(64), 0, (hipStream_t)stream, out3);
-  hipLaunchKernelGGL(pxl::k_coord_min, dim3(stride_blocks(n, 256, 2048)), dim3(256), 0,
-                     (hipStream_t)stream, coords, n, out3);
+  const unsigned nb = std::min(3 * stride_blocks(n, 256 * 4 * 3), (unsigned)pxl::kMinBlocks);  // a multiple of 3
+  hipLaunchKernelGGL(pxl::k_coord_min, dim3(nb), dim3(256), 0, (hipStream_t)stream, coords, n,
+                     (reinterpret_cast<uintptr_t>(coords) & 15u) == 0 ? 1 : 0, out3);
   return launched("pxl_coord_min");
 }
 
@@ -1147,19 +1225,37 @@ int pxl_tv_sumsq(const float* grid, int64_t X, int64_t Y, int64_t Z, double* sum
   return launched("pxl_tv_sumsq");
 }
 
-int pxl_tv_bwd(const float* grid, int64_t X, int64_t Y, int64_t Z, const double* sum_sq,
-               float weight, float* grad_grid, void* stream) {
+static int check_tv_grad(const float* grid, int64_t X, int64_t Y, int64_t Z, const double* sum_sq,
+                         const float* grad_grid) {
   int rc;
   if ((rc = pxl_host::check_dims(X, Y, Z)) ||
       (rc = need(grid && sum_sq && grad_grid, "grid, sum_sq and grad_grid required")) ||
       (rc = need(((reinterpret_cast<uintptr_t>(grid) | reinterpret_cast<uintptr_t>(grad_grid)) & 15u) == 0,
                  "grid and grad_grid must be 16-byte aligned")))
     return rc;
-  if (pxl::tv_units(X, Y, Z) > int64_t(0x7fffffff)) return fail(PXL_E_SIZE, "grid too large for pxl_tv_bwd");
-  hipLaunchKernelGGL(pxl::k_tv_bwd, dim3((unsigned)pxl::tv_units(X, Y, Z)), dim3(256), 0,
-                     (hipStream_t)stream, (const float4*)grid, Dims{X, Y, Z}, sum_sq, weight,
-                     reinterpret_cast<float4*>(grad_grid));
+  if (pxl::tv_units(X, Y, Z) > int64_t(0x7fffffff)) return fail(PXL_E_SIZE, "grid too large for the TV gradient");
+  return PXL_OK;
+}
+
+int pxl_tv_bwd(const float* grid, int64_t X, int64_t Y, int64_t Z, const double* sum_sq,
+               float weight, float* grad_grid, void* stream) {
+  int rc;
+  if ((rc = check_tv_grad(grid, X, Y, Z, sum_sq, grad_grid))) return rc;
+  hipLaunchKernelGGL(pxl::k_tv_bwd<false>, dim3((unsigned)pxl::tv_units(X, Y, Z, pxl::tv_bwd_slab(X, Y, Z))), dim3(256), 0,
+                     (hipStream_t)stream, (const float4*)grid, Dims{X, Y, Z}, pxl::tv_bwd_slab(X, Y, Z), sum_sq, weight,
+                     (const float*)nullptr, reinterpret_cast<float4*>(grad_grid));
   return launched("pxl_tv_bwd");
+}
+
+int pxl_tv_grad(const float* grid, int64_t X, int64_t Y, int64_t Z, const double* sum_sq, const float* weight,
+                float* grad_grid, void* stream) {
+  int rc;
+  if ((rc = check_tv_grad(grid, X, Y, Z, sum_sq, grad_grid)) || (rc = need(weight != nullptr, "weight is NULL")))
+    return rc;
+  hipLaunchKernelGGL(pxl::k_tv_bwd<true>, dim3((unsigned)pxl::tv_units(X, Y, Z, pxl::tv_bwd_slab(X, Y, Z))), dim3(256), 0, (hipStream_t)stream,
+                     (const float4*)grid, Dims{X, Y, Z}, pxl::tv_bwd_slab(X, Y, Z), sum_sq, 0.f, weight,
+                     reinterpret_cast<float4*>(grad_grid));
+  return launched("pxl_tv_grad");
 }
 
 int pxl_adam_tv_step(const float* param_in, float* param_out, float* grad, float* exp_avg,

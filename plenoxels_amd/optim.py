@@ -115,8 +115,13 @@ class _TVFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         grid, s = ctx.saved_tensors
-        grad = torch.zeros_like(grid, dtype=torch.float32)
-        tv_backward_(grid, s, float(g), grad)
+        grid = grid.contiguous()
+        grad = torch.empty_like(grid)
+        X, Y, Z = grid.shape[:3]
+        # the upstream gradient stays on the device: no synchronisation
+        w = g.to(device=grid.device, dtype=torch.float32).contiguous()
+        _lib.check(_lib.lib().pxl_tv_grad(_lib.ptr(grid), X, Y, Z, _lib.ptr(s), _lib.ptr(w), _lib.ptr(grad),
+                                          _lib.stream_handle(grid.device)))
         return grad
 
 

@@ -168,6 +168,16 @@ int pxl_train_step(const pxl_grid* grid, const pxl_march* march, const pxl_rays*
 int pxl_scaled_sum(const float* v, int64_t n, double scale, float* out, void* work, void* stream);
 int64_t pxl_scaled_sum_work_bytes(void);
 
+/* A training step's loss values in one launch, the same bits on every call: out4 (4 floats) =
+ *   { sq_scale * sum sq_err,  tv_weight * sqrt(*tv_sum_sq)  (tv_sum_sq NULL: 0),
+ *     beta * (sum ray_beta + beta_base) / n_samples  (ray_beta NULL: 0),  their float32 sum }
+ * with sq_err, ray_beta (n) as pxl_train_step writes them and sums and terms in FP64.  work: a
+ * device buffer of pxl_loss_terms_work_bytes, zeroed once and used by one call at a time. */
+int64_t pxl_loss_terms_work_bytes(void);
+int pxl_loss_terms(const float* sq_err, const float* ray_beta, const double* tv_sum_sq, int64_t n,
+                   double sq_scale, double tv_weight, double beta, double beta_base, double n_samples,
+                   float* out4, void* work, void* stream);
+
 /* pxl_scaled_sum without the caller's work buffer: the same kernel and the same bits, with its
  * partials and ticket in a scratch array the library keeps in each GPU's memory
  * (pxl_scaled_sum_noalloc_scratch_bytes() = 1 KiB per GPU, held until the process ends).  No
@@ -393,6 +403,14 @@ int pxl_tv_grad(const float* grid, int64_t X, int64_t Y, int64_t Z, const double
 int pxl_adam_step(float* param, const float* grad, float* exp_avg, float* exp_avg_sq,
                   float* grad_abs, int64_t n, double lr, double beta1, double beta2, double eps,
                   int64_t step, void* half_out, int32_t half_dtype, void* stream);
+
+/* pxl_avg_pool3d_bwd (overwriting) then pxl_adam_step, the same bits, without the full grid's
+ * gradient in memory: grad_out is the pooled grid's gradient, param, the moments, grad_abs and
+ * half_out the full (X,Y,Z,4) grid's; workspace of pxl_avg_pool3d_workspace_floats. */
+int pxl_adam_pooled_step(float* param, const float* grad_out, float* exp_avg, float* exp_avg_sq,
+                         float* grad_abs, int64_t X, int64_t Y, int64_t Z, int32_t k, int32_t s,
+                         double lr, double beta1, double beta2, double eps, int64_t step,
+                         void* half_out, int32_t half_dtype, float* workspace, void* stream);
 
 /* pxl_tv_bwd followed by pxl_adam_step in one pass over an (X,Y,Z,4) grid (scripts/train.py:
  * 163-168 and :180-184 for a step with the TV term): the total gradient grad + d(tv_weight *

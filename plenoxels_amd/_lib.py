@@ -133,6 +133,13 @@ SIGNATURES = {
                                   ctypes.c_float, c_void_p, c_void_p]),
     "pxl_tv_grad": (ctypes.c_int, [c_void_p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, c_void_p, c_void_p,
                                    c_void_p, c_void_p]),
+    "pxl_loss_terms_work_bytes": (ctypes.c_int64, []),
+    "pxl_loss_terms": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, ctypes.c_int64, *[ctypes.c_double] * 5, c_void_p,
+                                      c_void_p, c_void_p]),
+    "pxl_adam_pooled_step": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_int64,
+                                            ctypes.c_int64, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32,
+                                            ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double,
+                                            ctypes.c_int64, c_void_p, ctypes.c_int32, c_void_p, c_void_p]),
     "pxl_adam_step": (ctypes.c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_int64,
                                      ctypes.c_double, ctypes.c_double, ctypes.c_double, ctypes.c_double,
                                      ctypes.c_int64, c_void_p, ctypes.c_int32, c_void_p]),

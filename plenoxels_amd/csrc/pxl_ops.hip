@@ -646,6 +646,19 @@ __device__ __forceinline__ void store_half(void* half_out, int half_dtype, int64
     reinterpret_cast<_Float16*>(half_out)[i] = (_Float16)x;
 }
 
+__device__ __forceinline__ void store_half4(void* half_out, int half_dtype, int64_t i4, const float4& x) {
+  if (half_dtype == PXL_DTYPE_BF16) {
+    const uint32_t lo = to_bf16_rne(x.x) | ((uint32_t)to_bf16_rne(x.y) << 16);
+    const uint32_t hi = to_bf16_rne(x.z) | ((uint32_t)to_bf16_rne(x.w) << 16);
+    reinterpret_cast<uint2*>(half_out)[i4] = make_uint2(lo, hi);
+  } else {
+    store_half(half_out, half_dtype, 4 * i4 + 0, x.x);
+    store_half(half_out, half_dtype, 4 * i4 + 1, x.y);
+    store_half(half_out, half_dtype, 4 * i4 + 2, x.z);
+    store_half(half_out, half_dtype, 4 * i4 + 3, x.w);
+  }
+}
+
 // Elements [0, 4*n4) four at a time with 16-byte loads and stores (every pointer 16-byte
 // aligned), then the tail [4*n4, n) one at a time.
 __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
@@ -669,18 +682,7 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
       A = make_float4(A.x + fabsf(G.x), A.y + fabsf(G.y), A.z + fabsf(G.z), A.w + fabsf(G.w));
       reinterpret_cast<float4*>(gabs)[i] = A;
     }
-    if (half_out) {
-      if (half_dtype == PXL_DTYPE_BF16) {
-        const uint32_t lo = to_bf16_rne(P.x) | ((uint32_t)to_bf16_rne(P.y) << 16);
-        const uint32_t hi = to_bf16_rne(P.z) | ((uint32_t)to_bf16_rne(P.w) << 16);
-        reinterpret_cast<uint2*>(half_out)[i] = make_uint2(lo, hi);
-      } else {
-        store_half(half_out, half_dtype, 4 * i + 0, P.x);
-        store_half(half_out, half_dtype, 4 * i + 1, P.y);
-        store_half(half_out, half_dtype, 4 * i + 2, P.z);
-        store_half(half_out, half_dtype, 4 * i + 3, P.w);
-      }
-    }
+    if (half_out) store_half4(half_out, half_dtype, i, P);
   }
   PXL_GRID_STRIDE(j, n - 4 * n4) {
     const int64_t i = 4 * n4 + j;
@@ -692,6 +694,45 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
     p[i] = pi;
     if (gabs) gabs[i] += fabsf(gi);
     if (half_out) store_half(half_out, half_dtype, i, pi);
+  }
+}
+
+// k_adam on the gradient of a pooled grid: the last pass of the pooling adjoint (along z, from
+// d (X,Y,n_out)) is formed in registers by k_box_mean_adjoint's own sum, so the full grid's
+// gradient is neither written nor read back (32 of 160 bytes per cell).
+__global__ __launch_bounds__(256) void k_adam_pooled(float4* __restrict__ p, const float4* __restrict__ d,
+                                                     float4* __restrict__ m, float4* __restrict__ v,
+                                                     float4* __restrict__ gabs, uint32_t Z, uint32_t n_cells, int k,
+                                                     int s, uint32_t n_out, float w1, float beta2, float w2,
+                                                     float bc2_sqrt, float eps, float neg_step,
+                                                     void* __restrict__ half_out, int half_dtype) {
+  const float fk = (float)k;
+  for (uint32_t L = blockIdx.x * 256u + threadIdx.x; L < n_cells; L += gridDim.x * 256u) {
+    const uint32_t row = L / Z, z = L - row * Z;
+    const uint32_t lo = z + 1u <= (uint32_t)k ? 0u : (z - (uint32_t)k + (uint32_t)s) / (uint32_t)s;
+    const uint32_t hi = min(z / (uint32_t)s, n_out - 1u);
+    float4 G = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t o = lo; o <= hi; ++o) {
+      const float4 g = d[(size_t)row * n_out + o];
+      G.x += g.x;
+      G.y += g.y;
+      G.z += g.z;
+      G.w += g.w;
+    }
+    G = make_float4(G.x / fk, G.y / fk, G.z / fk, G.w / fk);
+    float4 P = p[L], M = m[L], V = v[L];
+    adam_elem(P.x, G.x, M.x, V.x, w1, beta2, w2, bc2_sqrt, eps, neg_step);
+    adam_elem(P.y, G.y, M.y, V.y, w1, beta2, w2, bc2_sqrt, eps, neg_step);
+    adam_elem(P.z, G.z, M.z, V.z, w1, beta2, w2, bc2_sqrt, eps, neg_step);
+    adam_elem(P.w, G.w, M.w, V.w, w1, beta2, w2, bc2_sqrt, eps, neg_step);
+    p[L] = P;
+    m[L] = M;
+    v[L] = V;
+    if (gabs) {
+      const float4 A = gabs[L];
+      gabs[L] = make_float4(A.x + fabsf(G.x), A.y + fabsf(G.y), A.z + fabsf(G.z), A.w + fabsf(G.w));
+    }
+    if (half_out) store_half4(half_out, half_dtype, L, P);
   }
 }
 
@@ -740,18 +781,7 @@ __global__ __launch_bounds__(256) void k_adam_tv(const float4* __restrict__ p_in
       A = make_float4(A.x + fabsf(G.x), A.y + fabsf(G.y), A.z + fabsf(G.z), A.w + fabsf(G.w));
       gabs[L] = A;
     }
-    if (half_out) {
-      if (half_dtype == PXL_DTYPE_BF16) {
-        const uint32_t lo = to_bf16_rne(Q.x) | ((uint32_t)to_bf16_rne(Q.y) << 16);
-        const uint32_t hi = to_bf16_rne(Q.z) | ((uint32_t)to_bf16_rne(Q.w) << 16);
-        reinterpret_cast<uint2*>(half_out)[L] = make_uint2(lo, hi);
-      } else {
-        store_half(half_out, half_dtype, 4 * L + 0, Q.x);
-        store_half(half_out, half_dtype, 4 * L + 1, Q.y);
-        store_half(half_out, half_dtype, 4 * L + 2, Q.z);
-        store_half(half_out, half_dtype, 4 * L + 3, Q.w);
-      }
-    }
+    if (half_out) store_half4(half_out, half_dtype, L, Q);
     Pm = P;
     P = Pp;
   }
@@ -804,6 +834,69 @@ __global__ __launch_bounds__(256) void k_scaled_sum(const float4* __restrict__ v
   p = wave_sum_f64(p);
   if (lane == 0) {
     out[0] = (float)(p * scale);
+    __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// A training step's loss values in one launch: out = {closs, tvloss, betaloss, their sum}.
+//   closs = sq_scale * sum sq;  tvloss = tv_weight * sqrt(tv_sum) (tv_sum NULL: 0);
+//   betaloss = beta * (sum bs + beta_base) / n_samples (bs NULL: 0), sums and terms in FP64.
+// The sums take k_scaled_sum's fixed order (workgroup strides, partials in index order); the last
+// workgroup to take a ticket finishes.  A 256^3 step with TV and beta ran ten torch kernels of
+// ~5 us for these scalars.
+struct LossTerms {
+  const float *sq, *bs;
+  const double* tv_sum;
+  int64_t n;
+  double sq_scale, tv_weight, beta, beta_base, n_samples;
+};
+
+__device__ __forceinline__ double strided_sum(const float* v, int64_t n, int64_t first, int64_t stride) {
+  double s = 0.0;
+#pragma unroll 8
+  for (int64_t i = first; i < n; i += stride) s += (double)v[i];
+  return s;
+}
+
+__global__ __launch_bounds__(256) void k_loss_terms(LossTerms T, float* __restrict__ out, double* __restrict__ partial,
+                                                    uint32_t* __restrict__ ticket) {
+  __shared__ double wsum[2][4];
+  __shared__ uint32_t last;
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t first = (int64_t)blockIdx.x * 256 + tid, stride = (int64_t)gridDim.x * 256;
+  const double a = wave_sum_f64(strided_sum(T.sq, T.n, first, stride));
+  const double b = T.bs ? wave_sum_f64(strided_sum(T.bs, T.n, first, stride)) : 0.0;
+  if (lane == 0) {
+    wsum[0][wave] = a;
+    wsum[1][wave] = b;
+  }
+  __syncthreads();
+  if (tid == 0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      partial[i * kSumBlocks + blockIdx.x] = (wsum[i][0] + wsum[i][1]) + (wsum[i][2] + wsum[i][3]);
+    __threadfence();  // the partials are visible device-wide before the ticket is taken
+    last = atomicAdd(ticket, 1u) == gridDim.x - 1u ? 1u : 0u;
+  }
+  __syncthreads();
+  if (last == 0u || wave != 0) return;
+  __threadfence();
+  double p[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    p[i] = lane < (int)gridDim.x ? __hip_atomic_load(partial + i * kSumBlocks + lane, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT)
+                                 : 0.0;
+    p[i] = wave_sum_f64(p[i]);
+  }
+  if (lane == 0) {
+    const float closs = (float)(p[0] * T.sq_scale);
+    const float tvloss = T.tv_sum ? (float)(T.tv_weight * sqrt(*T.tv_sum)) : 0.f;
+    const float betaloss = T.bs ? (float)(T.beta * (p[1] + T.beta_base) / T.n_samples) : 0.f;
+    out[0] = closs;
+    out[1] = tvloss;
+    out[2] = betaloss;
+    out[3] = (closs + tvloss) + betaloss;
     __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
@@ -1112,6 +1205,19 @@ int pxl_avg_pool3d(const float* grid, int64_t X, int64_t Y, int64_t Z, int32_t k
   return launched("pxl_avg_pool3d");
 }
 
+// The pooling adjoint along x and y: (X,Y,oz) in the workspace.
+static const float4* pool_adjoint_xy(const float* grad_out, int64_t X, int64_t Y, int64_t Z, int32_t k, int32_t s,
+                                     float* workspace, hipStream_t st) {
+  const int64_t ox = (X - k) / s + 1, oy = (Y - k) / s + 1, oz = (Z - k) / s + 1;
+  float4* d = reinterpret_cast<float4*>(workspace);  // (X, Y, oz)
+  float4* c = d + X * Y * oz;                         // (X, oy, oz)
+  hipLaunchKernelGGL(pxl::k_box_mean_adjoint, dim3(stride_blocks(X * oy * oz, 256)), dim3(256), 0, st,
+                     (const float4*)grad_out, (int64_t)1, X, oy * oz, k, s, ox, 0, c);
+  hipLaunchKernelGGL(pxl::k_box_mean_adjoint, dim3(stride_blocks(X * Y * oz, 256)), dim3(256), 0, st,
+                     (const float4*)c, X, Y, oz, k, s, oy, 0, d);
+  return d;
+}
+
 int pxl_avg_pool3d_bwd(const float* grad_out, int64_t X, int64_t Y, int64_t Z, int32_t k,
                        int32_t s, float* grad_grid, int32_t accumulate, float* workspace, void* stream) {
   int rc;
@@ -1119,16 +1225,11 @@ int pxl_avg_pool3d_bwd(const float* grad_out, int64_t X, int64_t Y, int64_t Z, i
       (rc = need(grad_out && grad_grid && workspace, "pointers required")) ||
       (rc = need(k >= 1 && s >= 1 && k <= X && k <= Y && k <= Z, "need 1 <= k <= dims, s >= 1")))
     return rc;
-  const int64_t ox = (X - k) / s + 1, oy = (Y - k) / s + 1, oz = (Z - k) / s + 1;
-  float4* d = reinterpret_cast<float4*>(workspace);  // (X, Y, oz)
-  float4* c = d + X * Y * oz;                         // (X, oy, oz)
+  const int64_t oz = (Z - k) / s + 1;
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(pxl::k_box_mean_adjoint, dim3(stride_blocks(X * oy * oz, 256)), dim3(256), 0, st,
-                     (const float4*)grad_out, (int64_t)1, X, oy * oz, k, s, ox, 0, c);
-  hipLaunchKernelGGL(pxl::k_box_mean_adjoint, dim3(stride_blocks(X * Y * oz, 256)), dim3(256), 0, st,
-                     (const float4*)c, X, Y, oz, k, s, oy, 0, d);
+  const float4* d = pool_adjoint_xy(grad_out, X, Y, Z, k, s, workspace, st);
   hipLaunchKernelGGL(pxl::k_box_mean_adjoint, dim3(stride_blocks(X * Y * Z, 256)), dim3(256), 0, st,
-                     (const float4*)d, X * Y, Z, (int64_t)1, k, s, oz, accumulate ? 1 : 0, (float4*)grad_grid);
+                     d, X * Y, Z, (int64_t)1, k, s, oz, accumulate ? 1 : 0, (float4*)grad_grid);
   return launched("pxl_avg_pool3d_bwd");
 }
 
@@ -1145,6 +1246,21 @@ int pxl_scaled_sum(const float* v, int64_t n, double scale, float* out, void* wo
   hipLaunchKernelGGL(pxl::k_scaled_sum, dim3(pxl::kSumBlocks), dim3(256), 0, (hipStream_t)stream,
                      reinterpret_cast<const float4*>(v), v, n, scale, out, partial, ticket);
   return launched("pxl_scaled_sum");
+}
+
+int64_t pxl_loss_terms_work_bytes(void) { return 2 * pxl::kSumBlocks * (int64_t)sizeof(double) + 16; }
+
+int pxl_loss_terms(const float* sq_err, const float* ray_beta, const double* tv_sum_sq, int64_t n, double sq_scale,
+                   double tv_weight, double beta, double beta_base, double n_samples, float* out4, void* work,
+                   void* stream) {
+  if (n < 0) return fail(PXL_E_INVALID, "n must be >= 0");
+  if (!out4 || !work || (n > 0 && !sq_err)) return fail(PXL_E_INVALID, "sq_err, out4 and work are required");
+  if (reinterpret_cast<uintptr_t>(work) % 16 != 0) return fail(PXL_E_INVALID, "work must be 16-byte aligned");
+  double* partial = reinterpret_cast<double*>(work);
+  hipLaunchKernelGGL(pxl::k_loss_terms, dim3(pxl::kSumBlocks), dim3(256), 0, (hipStream_t)stream,
+                     pxl::LossTerms{sq_err, ray_beta, tv_sum_sq, n, sq_scale, tv_weight, beta, beta_base, n_samples},
+                     out4, partial, reinterpret_cast<uint32_t*>(partial + 2 * pxl::kSumBlocks));
+  return launched("pxl_loss_terms");
 }
 
 int64_t pxl_scaled_sum_noalloc_scratch_bytes(void) { return pxl::kNoAllocScratchBytes; }
@@ -1289,6 +1405,35 @@ int pxl_adam_tv_step(const float* param_in, float* param_out, float* grad, float
                      tv_sum_sq, tv_weight, (float)(1.0 - beta1), (float)beta2, (float)(1.0 - beta2), bc2_sqrt,
                      (float)eps, neg_step, half_out, half_dtype, zero_grad ? 1 : 0);
   return launched("pxl_adam_tv_step");
+}
+
+int pxl_adam_pooled_step(float* param, const float* grad_out, float* exp_avg, float* exp_avg_sq, float* grad_abs,
+                         int64_t X, int64_t Y, int64_t Z, int32_t k, int32_t s, double lr, double beta1, double beta2,
+                         double eps, int64_t step, void* half_out, int32_t half_dtype, float* workspace,
+                         void* stream) {
+  int rc;
+  auto al16 = [](const void* q) { return q == nullptr || (reinterpret_cast<uintptr_t>(q) & 15u) == 0; };
+  if ((rc = pxl_host::check_dims(X, Y, Z)) ||
+      (rc = need(param && grad_out && exp_avg && exp_avg_sq && workspace,
+                 "param, grad_out, moments and workspace required")) ||
+      (rc = need(k >= 1 && s >= 1 && k <= X && k <= Y && k <= Z, "need 1 <= k <= dims, s >= 1")) ||
+      (rc = need(step >= 1, "step counts from 1")) ||
+      (rc = need(!half_out || half_dtype == PXL_DTYPE_BF16 || half_dtype == PXL_DTYPE_F16,
+                 "half_dtype must be PXL_DTYPE_BF16 or PXL_DTYPE_F16")) ||
+      (rc = need(al16(param) && al16(grad_out) && al16(exp_avg) && al16(exp_avg_sq) && al16(grad_abs) &&
+                     al16(workspace) && (half_out == nullptr || (reinterpret_cast<uintptr_t>(half_out) & 7u) == 0),
+                 "float arrays must be 16-byte aligned (half_out 8-byte)")))
+    return rc;
+  const float4* d = pool_adjoint_xy(grad_out, X, Y, Z, k, s, workspace, (hipStream_t)stream);
+  const double bc1 = 1.0 - std::pow(beta1, (double)step);
+  const double bc2 = 1.0 - std::pow(beta2, (double)step);
+  const int64_t n = X * Y * Z;
+  hipLaunchKernelGGL(pxl::k_adam_pooled, dim3(stride_blocks(n, 256)), dim3(256), 0, (hipStream_t)stream,
+                     reinterpret_cast<float4*>(param), d, reinterpret_cast<float4*>(exp_avg),
+                     reinterpret_cast<float4*>(exp_avg_sq), reinterpret_cast<float4*>(grad_abs), (uint32_t)Z, (uint32_t)n,
+                     k, s, (uint32_t)((Z - k) / s + 1), (float)(1.0 - beta1), (float)beta2, (float)(1.0 - beta2),
+                     (float)std::pow(bc2, 0.5), (float)eps, (float)(-(lr / bc1)), half_out, half_dtype);
+  return launched("pxl_adam_pooled_step");
 }
 
 int pxl_adam_step(float* param, const float* grad, float* exp_avg, float* exp_avg_sq,

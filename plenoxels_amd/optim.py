@@ -12,6 +12,7 @@ the three axes), summed on the device in FP64.
 import torch
 
 from . import _lib
+from .grid_functions import _pool_workspace
 
 _HALF = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16}
 
@@ -67,6 +68,20 @@ def adam_step_(param, grad, exp_avg, exp_avg_sq, step, *, lr, betas=(0.9, 0.999)
         param.numel(), float(lr), float(betas[0]), float(betas[1]), float(eps), int(step),
         _lib.ptr(half_out), _HALF[half_out.dtype] if half_out is not None else 0,
         _lib.stream_handle(param.device)))
+
+
+def adam_pooled_step_(param, grad_out, k, stride, exp_avg, exp_avg_sq, step, *, lr, betas=(0.9, 0.999), eps=1e-8,
+                      grad_abs=None, half_out=None):
+    """pool_backward_ of the pooled grid's gradient grad_out into a full gradient, then adam_step_
+    with it, in one pass over the grid (pxl_adam_pooled_step): the same bits, and the full
+    gradient is never written."""
+    X, Y, Z = (int(v) for v in param.shape[:3])
+    go = grad_out.float().contiguous()
+    ws = _pool_workspace((X, Y, Z), k, stride, param.device)
+    _lib.check(_lib.lib().pxl_adam_pooled_step(
+        _lib.ptr(param), _lib.ptr(go), _lib.ptr(exp_avg), _lib.ptr(exp_avg_sq), _lib.ptr(grad_abs), X, Y, Z, int(k),
+        int(stride), float(lr), float(betas[0]), float(betas[1]), float(eps), int(step), _lib.ptr(half_out),
+        _HALF[half_out.dtype] if half_out is not None else 0, _lib.ptr(ws), _lib.stream_handle(param.device)))
 
 
 def adam_tv_step_(param_in, param_out, grad, exp_avg, exp_avg_sq, step, *, tv_sumsq, tv_weight, lr,

@@ -435,6 +435,26 @@ class LossMean:
         return out
 
 
+class LossTerms:
+    """The loss values of a training step (scripts/train.py:156-174) from its per-ray partials and
+    the TV sum, on the device in one launch (pxl_loss_terms).  Holds the call's small work buffer:
+    use one instance per stream."""
+
+    def __init__(self, device):
+        self.work = torch.zeros(int(_lib.lib().pxl_loss_terms_work_bytes()), dtype=torch.uint8, device=device)
+
+    def __call__(self, ray_sq_err, n_rays, *, tv_sumsq=None, tv_weight=0.0, ray_beta=None, beta=0.0, n_samples=0):
+        """float32 (4,): mean squared error, tv_weight * TV, beta term (0 where not given), sum."""
+        if n_rays <= 0:
+            raise ValueError("n_rays must be positive")
+        out = torch.empty(4, dtype=torch.float32, device=self.work.device)
+        _lib.check(_lib.lib().pxl_loss_terms(
+            _lib.ptr(ray_sq_err), _lib.ptr(ray_beta), _lib.ptr(tv_sumsq), ray_sq_err.shape[0], 1.0 / (4.0 * n_rays),
+            float(tv_weight), float(beta), n_samples * beta_term_zero(), float(n_samples), _lib.ptr(out),
+            _lib.ptr(self.work), _lib.stream_handle(out.device)))
+        return out
+
+
 def fill_(t, value=0.0):
     """In-place fill of a contiguous float32 device tensor with the library's fill kernel."""
     if t.dtype != torch.float32 or not t.is_contiguous() or not t.is_cuda:

@@ -20,10 +20,10 @@ import torch
 
 from . import _lib
 from .checkpoint import save_grid
-from .grid_functions import average_pool3d_grid, pool_backward_
-from .optim import adam_step_, adam_tv_step_, tv_backward_, tv_sumsq
-from .render import (CameraRays, CornerBlockPair, LossMean, MarchConfig, alpha_occupancy, beta_term_zero, blocks_reduce,
-                     fill_, train_step)
+from .grid_functions import average_pool3d_grid
+from .optim import adam_pooled_step_, adam_step_, adam_tv_step_, tv_backward_, tv_sumsq
+from .render import (CameraRays, CornerBlockPair, LossTerms, MarchConfig, alpha_occupancy, blocks_reduce, fill_,
+                     train_step)
 
 RECEPTIVE_FIELDS = [i for i in range(93, 2, -2) if i % 2 != 0]  # scripts/train.py:91
 STEPS_PER_FIELD = 5                                              # scripts/train.py:92
@@ -118,7 +118,7 @@ class Trainer:
         self.n_rays = n
         self.cam_ids = torch.repeat_interleave(torch.arange(self.B, dtype=torch.int32, device=self.dev), self.R)
         self.sq = torch.empty(n, device=self.dev)
-        self.loss_mean = LossMean(self.dev)
+        self.loss_terms = LossTerms(self.dev)
         self.bsum = torch.empty(n, device=self.dev)
         self.tvs = torch.zeros(1, dtype=torch.float64, device=self.dev)
         self._grid_next = None  # second FP32 grid of the fused TV + Adam update (allocated on first use)
@@ -204,30 +204,26 @@ class Trainer:
                        overwrite=True, clear=pair.other if pair else None)
         if pair:
             pair.flip()
-        closs = self.loss_mean(self.sq, n_rays)
-        out = {"closs": closs}
-        loss = closs
         # full-grid steps with the TV term fold its backward into the Adam pass (pxl_adam_tv_step,
         # the same bits), which writes the updated grid into a second buffer
         fused_tv = use_tv and not pooled
+        if use_tv and not tv_with_occ:
+            tv_sumsq(tv_grid, out=self.tvs)
+        if use_tv and pooled:
+            tv_backward_(tv_grid, self.tvs, self.tv, grad)
+        use_beta = self.beta > 0
+        terms = self.loss_terms(self.sq, n_rays, tv_sumsq=self.tvs if use_tv else None, tv_weight=self.tv,
+                                ray_beta=self.bsum if use_beta else None, beta=self.beta, n_samples=n_rays * self.S)
+        out = {"closs": terms[0]}
         if use_tv:
-            if not tv_with_occ:
-                tv_sumsq(tv_grid, out=self.tvs)
-            if not fused_tv:
-                tv_backward_(tv_grid, self.tvs, self.tv, grad)
-            tvl = (self.tv * torch.sqrt(self.tvs)).float().reshape(())
-            out["tvloss"] = tvl
-            loss = loss + tvl
-        if self.beta > 0:
-            n_s = n_rays * self.S
-            bl = self.beta * (self.bsum.sum() + n_s * beta_term_zero()) / n_s
-            out["betaloss"] = bl
-            loss = loss + bl
-        if pooled:  # the full grid's gradient, every cell written
-            pool_backward_(grad, (X, Y, Z), k, max(1, k // 4), self.grad, accumulate=False)
-            self._grad_zero = False
+            out["tvloss"] = terms[1]
+        if use_beta:
+            out["betaloss"] = terms[2]
         self.step_count += 1
-        if fused_tv:
+        if pooled:  # the pooling backward is part of the Adam pass: self.grad is neither read nor written
+            adam_pooled_step_(self.grid, grad, k, max(1, k // 4), self.exp_avg, self.exp_avg_sq, self.step_count,
+                              lr=self.lr, grad_abs=self.grad_abs, half_out=self.render_copy)
+        elif fused_tv:
             if self._grid_next is None:
                 self._grid_next = torch.empty_like(self.grid)
             # the pass leaves the gradient zero for the next step (no separate zero-fill)
@@ -239,7 +235,7 @@ class Trainer:
         else:
             adam_step_(self.grid, self.grad, self.exp_avg, self.exp_avg_sq, self.step_count, lr=self.lr,
                        grad_abs=self.grad_abs, half_out=self.render_copy)
-        out["loss"] = loss
+        out["loss"] = terms[3]
         return out
 
     def save(self, save_path, device_name):

@@ -439,25 +439,25 @@ __device__ __forceinline__ bool classify(const KParams& P, const Ray& R, int k) 
   return inb & (((P.occ[b.word] >> b.shift) & 1u) != 0u);
 }
 
-// classify() for NC chunks of each of NR rays (sample k = 64c + lane + 1 of ray r): every sample
+// classify() for chunks c0 .. c0 + NC - 1 of each of NR rays (sample k = 64c + lane + 1 of ray r): every sample
 // is placed first (the division mode chosen once, outside the loops), then all occupancy words
 // are loaded back to back and only then tested, so the loads of all chunks share one memory
 // round trip.  kp[r][c]: in the grid, occupied and k <= n_samples.
 template <int INTERP, int NR, int NC>
 __device__ __forceinline__ void classify_chunks(const KParams& P, const Ray (&R)[NR], int lane,
-                                                bool (&kp)[NR][NC]) {
+                                                bool (&kp)[NR][NC], int c0 = 0) {
   OccBit ob[NR][NC];
   bool inb[NR][NC];
   if (P.exact_div) {
 #pragma unroll
     for (int r = 0; r < NR; ++r)
 #pragma unroll
-      for (int c = 0; c < NC; ++c) inb[r][c] = locate<INTERP, true>(P, R[r], (c << 6) + lane + 1, ob[r][c]);
+      for (int c = 0; c < NC; ++c) inb[r][c] = locate<INTERP, true>(P, R[r], ((c0 + c) << 6) + lane + 1, ob[r][c]);
   } else {
 #pragma unroll
     for (int r = 0; r < NR; ++r)
 #pragma unroll
-      for (int c = 0; c < NC; ++c) inb[r][c] = locate<INTERP, false>(P, R[r], (c << 6) + lane + 1, ob[r][c]);
+      for (int c = 0; c < NC; ++c) inb[r][c] = locate<INTERP, false>(P, R[r], ((c0 + c) << 6) + lane + 1, ob[r][c]);
   }
   if (P.occ != nullptr) {
     uint32_t w[NR][NC];
@@ -473,7 +473,7 @@ __device__ __forceinline__ void classify_chunks(const KParams& P, const Ray (&R)
 #pragma unroll
   for (int r = 0; r < NR; ++r)
 #pragma unroll
-    for (int c = 0; c < NC; ++c) kp[r][c] = inb[r][c] & ((c << 6) + lane + 1 <= P.n_samples);
+    for (int c = 0; c < NC; ++c) kp[r][c] = inb[r][c] & (((c0 + c) << 6) + lane + 1 <= P.n_samples);
 }
 
 // torch.clamp(v, 0, 1): NaN stays NaN (v_med3 alone would return a bound)

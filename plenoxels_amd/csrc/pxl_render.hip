@@ -529,17 +529,25 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 
   const float4 tgt1 = !has1 ? tgt0
                     : targets ? reinterpret_cast<const float4*>(targets)[ray0 + 1] : camera_target(P, R1);
   const Ray RR[2] = {R0, R1};
-  bool kp[2][NG];
-  classify_chunks<INTERP, 2, NG>(P, RR, lane, kp);
+  // chunks classified together: all of both rays (one memory round trip), except where nearest
+  // lookup has eight, which leaves four waves per SIMD for them (100000 rays x 320 samples: 133 us
+  // together, 112 one by one; trilinear, bound by its gathers and scatter, 415 and 449)
+  constexpr int kBatch = NG == 8 && INTERP == PXL_INTERP_NEAREST ? 1 : NG;
   int n0 = 0, n1 = 0;
+  for (int c0 = 0; c0 < NG; c0 += kBatch) {
+    if (kBatch < NG && (c0 << 6) >= P.n_samples) break;
+    bool kp[2][kBatch];
+    classify_chunks<INTERP, 2, kBatch>(P, RR, lane, kp, c0);
 #pragma unroll
-  for (int c = 0; c < NG; ++c) {
-    const bool k1 = kp[1][c] & has1;
-    const uint64_t km0 = __ballot(kp[0][c]), km1 = __ballot(k1);
-    if (kp[0][c]) list0[n0 + lane_rank(km0)] = (c << 6) + lane + 1;
-    if (k1) list1[n1 + lane_rank(km1)] = (c << 6) + lane + 1;
-    n0 += __popcll(km0);
-    n1 += __popcll(km1);
+    for (int c = 0; c < kBatch; ++c) {
+      const bool k1 = kp[1][c] & has1;
+      const int k = ((c0 + c) << 6) + lane + 1;
+      const uint64_t km0 = __ballot(kp[0][c]), km1 = __ballot(k1);
+      if (kp[0][c]) list0[n0 + lane_rank(km0)] = k;
+      if (k1) list1[n1 + lane_rank(km1)] = k;
+      n0 += __popcll(km0);
+      n1 += __popcll(km1);
+    }
   }
   wave_lds_sync();
   const uint32_t first = (uint32_t)(ray0 - P.ray_offset);
@@ -559,9 +567,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 
   if (BIN && lane == 0) B.n_runs[first >> 1] = cur.n;
 }
 
-// Forward of two rays per wavefront for S <= 64 * NG: k_train_pair's classification (the
-// occupancy loads of all chunks of both rays in flight at once; a chunk at a time, each load
-// waited for the previous) and its half-wave group when each ray keeps at most 32 samples, else
+// Forward of two rays per wavefront for S <= 64 * NG: both rays classified together (up to two
+// chunks in one round trip; above 128 samples a chunk of each at a time, as many as the sample count
+// needs -- all eight in flight took 114 registers and 328 us where the loop takes 229, an 600x600
+// view with 331 nearest samples) and k_train_pair's half-wave group when each ray keeps at most 32 samples, else
 // the rays' groups one after the other.  Every value is formed by the operation tree of
 // forward_sweep, so outputs and aux are the same bits.
 // 800x800 view of a 256^3 FP16 grid with ~5% occupancy, 256 trilinear samples: 663 us with
@@ -604,6 +613,7 @@ __device__ __forceinline__ void fwd_ray(const KParams& P, const Ray& R, int64_t 
 template <int DT, int INTERP, int NG>
 __global__ __launch_bounds__(kBlock) void k_render_pair(KParams P, float* __restrict__ out, float* __restrict__ aux) {
   __shared__ int s_list[kWavesPerBlock][2][kWave * NG];
+  constexpr int kBatch = NG <= 2 ? NG : 1;  // chunks classified together
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t ray0 = P.ray_offset + 2 * ((int64_t)blockIdx.x * kWavesPerBlock + wave);
@@ -615,17 +625,21 @@ __global__ __launch_bounds__(kBlock) void k_render_pair(KParams P, float* __rest
   setup_ray(P, ray0, RR[0]);
   if (has1) setup_ray(P, ray0 + 1, RR[1]);
   else RR[1] = RR[0];
-  bool kp[2][NG];
-  classify_chunks<INTERP, 2, NG>(P, RR, lane, kp);
   int n0 = 0, n1 = 0;
+  for (int c0 = 0; c0 < NG; c0 += kBatch) {
+    if (kBatch < NG && (c0 << 6) >= P.n_samples) break;
+    bool kp[2][kBatch];
+    classify_chunks<INTERP, 2, kBatch>(P, RR, lane, kp, c0);
 #pragma unroll
-  for (int c = 0; c < NG; ++c) {
-    const bool k1 = kp[1][c] & has1;
-    const uint64_t km0 = __ballot(kp[0][c]), km1 = __ballot(k1);
-    if (kp[0][c]) list0[n0 + lane_rank(km0)] = (c << 6) + lane + 1;
-    if (k1) list1[n1 + lane_rank(km1)] = (c << 6) + lane + 1;
-    n0 += __popcll(km0);
-    n1 += __popcll(km1);
+    for (int c = 0; c < kBatch; ++c) {
+      const bool k1 = kp[1][c] & has1;
+      const int k = ((c0 + c) << 6) + lane + 1;
+      const uint64_t km0 = __ballot(kp[0][c]), km1 = __ballot(k1);
+      if (kp[0][c]) list0[n0 + lane_rank(km0)] = k;
+      if (k1) list1[n1 + lane_rank(km1)] = k;
+      n0 += __popcll(km0);
+      n1 += __popcll(km1);
+    }
   }
   wave_lds_sync();
   if (n0 > 32 || n1 > 32) {

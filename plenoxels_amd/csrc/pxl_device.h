@@ -665,6 +665,54 @@ __device__ __forceinline__ int merge_nearest_runs(int lane, int ns, uint32_t* s_
   return __popcll(tails);
 }
 
+// A workgroup's cell sums (nearest lookup, bundles of neighbouring rays): an open-addressed table
+// of cells in LDS with float64 sums of their four channels (ds_add_f32 takes ~195 clocks per wave
+// instruction on gfx950, ds_add_f64 9 to 41).
+constexpr uint32_t kSumSlots = 512, kSumEmpty = 0xffffffffu, kSumProbes = 8;
+
+__device__ __forceinline__ uint32_t* sum_keys() {
+  __shared__ uint32_t s_keys[kSumSlots];
+  return s_keys;
+}
+
+__device__ __forceinline__ double* sum_vals() {
+  __shared__ double s_vals[kSumSlots * 4];
+  return s_vals;
+}
+
+// Items 0 .. n-1 (n <= 64, cells in s_cell, which is overwritten) into the table; an item that finds
+// no slot within kProbes goes straight to grad.  Four lanes per item, as flush_cells.
+__device__ __forceinline__ void sum_cells(int lane, int n, float* grad, uint32_t* s_cell, const float* sv) {
+  uint32_t* keys = sum_keys();
+  double* vals = sum_vals();
+  constexpr uint32_t kInTable = 0x80000000u;  // cell indices stay below 2^31
+  if (lane < n) {
+    const uint32_t cell = s_cell[lane];
+    uint32_t h = (cell * 2654435761u) >> 23;  // the top nine bits: kSumSlots = 512
+    for (uint32_t p = 0; p < kSumProbes; ++p) {
+      const uint32_t was = atomicCAS(keys + h, kSumEmpty, cell);
+      if (was == kSumEmpty || was == cell) {
+        s_cell[lane] = h | kInTable;
+        break;
+      }
+      h = (h + 1u) & (kSumSlots - 1u);
+    }
+  }
+  wave_lds_sync();
+  const int ch = lane & 3;
+  for (int base = 0; base < n; base += kWave / 4) {
+    const int it = base + (lane >> 2);
+    if (it < n) {
+      const float v = sv[4 * it + ch];
+      const uint32_t c = s_cell[it];
+      if (v != 0.f) {
+        if (c & kInTable) unsafeAtomicAdd(vals + (c & ~kInTable) * 4u + ch, (double)v);
+        else atomic_add_f32(grad + (size_t)c * 4u + ch, v);
+      }
+    }
+  }
+}
+
 // Items 0 .. n-1 added to grad, four lanes per item: one memory request per cell.
 __device__ __forceinline__ void flush_cells(int lane, int n, float* grad, const uint32_t* s_cell, const float* sv) {
   const int ch = lane & 3;
@@ -680,7 +728,8 @@ __device__ __forceinline__ void flush_cells(int lane, int n, float* grad, const 
 template <int INTERP, bool RUNS = false>
 __device__ __forceinline__ void scatter_chunk(const KParams& P, const Ray& R, int lane, int k,
                                               bool keep, uint32_t clip, const float4& gv,
-                                              float* grad, uint32_t* s_cell, float4* s_val) {
+                                              float* grad, uint32_t* s_cell, float4* s_val,
+                                              bool sums = false) {
   constexpr int NI = ScatterItems<INTERP>::kPerSample;
   constexpr int NS = ScatterItems<INTERP>::kStageSamples;
   const uint64_t km = __ballot(keep);
@@ -715,7 +764,12 @@ __device__ __forceinline__ void scatter_chunk(const KParams& P, const Ray& R, in
         }
       }
     }
-    if (!by_runs) flush_cells(lane, n, grad, s_cell, sv);
+    bool summed = false;
+    if constexpr (RUNS && INTERP == PXL_INTERP_NEAREST) {
+      summed = sums;
+      if (summed) sum_cells(lane, n, grad, s_cell, sv);
+    }
+    if (!by_runs && !summed) flush_cells(lane, n, grad, s_cell, sv);
     wave_lds_sync();
   }
 }

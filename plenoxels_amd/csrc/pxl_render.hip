@@ -186,7 +186,7 @@ __device__ __forceinline__ void reverse_chunk(const KParams& P, const Ray& R, in
     if (beta_scale != 0.f) gv.w += beta_scale * beta_dloss(v.w);
   }
   if constexpr (BIN) emit_chunk(P, B, R, lane, k, keep, gv, cur);
-  else scatter_chunk<INTERP, RUNS>(P, R, lane, k, keep, clip, gv, grad, s_cell, s_val);
+  else scatter_chunk<INTERP, RUNS>(P, R, lane, k, keep, clip, gv, grad, s_cell, s_val, cur.sums);
   Qn = make_float4(readlane(f.a0, 0), readlane(f.a1, 0), readlane(f.a2, 0), readlane(f.a3, 0));
 }
 
@@ -249,7 +249,7 @@ __device__ __forceinline__ void reverse_sweep(const KParams& P, const Ray& R, in
 // The cursor of a wave whose first ray is `ray` (local index within the launch) in a region of
 // `rays` rays.
 __device__ __forceinline__ BinCursor bin_cursor(const KParams& P, const Bins& B, uint32_t ray, uint32_t rays) {
-  return BinCursor{ray * (uint32_t)P.n_samples, ray / rays * B.run_cap, 0u};
+  return BinCursor{ray * (uint32_t)P.n_samples, ray / rays * B.run_cap, 0u, false};
 }
 
 template <int DT, int INTERP, bool BIN>
@@ -296,7 +296,8 @@ struct LossParams {
 // -- dense grids, whose rays keep runs of samples in one cell (64^3, 32768 rays x 128 samples into
 // corner blocks: 330 -> 243 us) -- and not for sparse scenes, whose samples rarely share a cell
 // (sparse256 spills and takes the flush in none of its stages).  Above 256 samples per ray (three
-// waves per SIMD) it is always there.
+// waves per SIMD) it is always there.  For nearest lookup RUN stands for the cell sums of bundles
+// of rays (k_train_pair), again where no occupancy is given.
 template <int DT, int INTERP, int NG, bool BIN, bool RUN>
 __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP, const Ray& R,
                                           int64_t ray, const float4& tgt, const int* list, int nk,
@@ -501,23 +502,17 @@ __device__ __forceinline__ void train_half_pair(const KParams& P, const LossPara
     if (LP.beta_scale != 0.f) gv.w += LP.beta_scale * beta_dloss(V.w);
   }
   if constexpr (BIN) emit_chunk(P, B, R, lane, k, proc, gv, cur);
-  else scatter_chunk<INTERP, RUN>(P, R, lane, k, proc, CL, gv, grad, s_cell, s_val);
+  else scatter_chunk<INTERP, RUN>(P, R, lane, k, proc, CL, gv, grad, s_cell, s_val, cur.sums);
 }
 
+// One wave's pair of rays (ray0 < n_rays); mem: the wave's LDS,
+// [ray 0's list, then the scatter staging area | ray 1's list].
 template <int DT, int INTERP, int NG, bool BIN, bool RUN>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 && DT != PXL_DTYPE_F16 && !RUN ? 5 : 1))) void k_train_pair(KParams P, LossParams LP,
-                                                        float* __restrict__ out,
-                                                        float* __restrict__ grad, Bins B) {
-  // per wave: [ray 0's list, then the scatter staging area | ray 1's list]
+__device__ __forceinline__ void train_pair(const KParams& P, const LossParams& LP, int64_t ray0, int lane,
+                                           unsigned char* mem, float* __restrict__ out, float* __restrict__ grad,
+                                           const Bins& B, BinCursor& cur) {
   using L = WaveLds<INTERP, kWave * NG, BIN>;
-  constexpr int kList1 = kWave * NG * 4;
-  __shared__ __align__(16) unsigned char s_mem[kWavesPerBlock][L::kBytes + kList1];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int64_t ray0 = P.ray_offset + 2 * ((int64_t)blockIdx.x * kWavesPerBlock + wave);
-  if (ray0 >= P.n_rays) return;
   const bool has1 = ray0 + 1 < P.n_rays;
-  unsigned char* mem = s_mem[wave];
   int* list0 = L::list(mem);
   int* list1 = reinterpret_cast<int*>(mem + L::kBytes);
   Ray R0, R1;
@@ -551,7 +546,6 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 
   }
   wave_lds_sync();
   const uint32_t first = (uint32_t)(ray0 - P.ray_offset);
-  BinCursor cur{};
   if constexpr (BIN) cur = bin_cursor(P, B, first, 2u);
   if (n0 <= 32 && n1 <= 32) {
     train_half_pair<DT, INTERP, NG, BIN, RUN>(P, LP, R0, R1, ray0, has1, tgt0, tgt1, list0, n0, list1, n1, lane,
@@ -565,6 +559,64 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 
                                      grad, B, cur);
   }
   if (BIN && lane == 0) B.n_runs[first >> 1] = cur.n;
+}
+
+
+// Whether a workgroup's rays are neighbours: its first and last ray stay within eight cells of each
+// other along their samples (their distance is largest at one of the ends).  Within four
+// cells only, a 400x400 view of a 256^3 grid (200 samples) misses the sums: 953 us, and 730 with them.
+__device__ __forceinline__ bool is_bundle(const KParams& P) {
+  const int64_t a = P.ray_offset + (int64_t)blockIdx.x * 2 * kWavesPerBlock;
+  const int64_t b = min(a + 2 * kWavesPerBlock, P.n_rays) - 1;
+  Ray A, Z;
+  setup_ray(P, a, A);
+  setup_ray(P, b, Z);
+  const float ts[2] = {P.delta + P.near, P.delta * (float)P.n_samples + P.near};
+  float most = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    most = fmaxf(most, fmaxf(fabsf((A.ox - Z.ox) + (A.dx - Z.dx) * ts[i]),
+                             fmaxf(fabsf((A.oy - Z.oy) + (A.dy - Z.dy) * ts[i]),
+                                   fabsf((A.oz - Z.oz) + (A.dz - Z.dz) * ts[i]))));
+  return most <= 8.f * P.pd;
+}
+
+// Nearest lookup of a dense grid (RUN) adds ~140 runs of samples per ray; where a workgroup's
+// eight rays are neighbours (whole images, even spreads) they reach the same cells, so their sums
+// are formed in LDS first and added once: 128^3, one 800x800 view x 256 samples: 3.76 -> 1.54
+// ms.  Other workgroups add their runs themselves, at the speed they had (100000 random rays of 30
+// views x 256 samples, 128^3: 443 and 444 us).
+template <int DT, int INTERP, int NG, bool BIN, bool RUN>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 && DT != PXL_DTYPE_F16 && !RUN ? 5 : 1))) void k_train_pair(KParams P, LossParams LP,
+                                                        float* __restrict__ out,
+                                                        float* __restrict__ grad, Bins B) {
+  // per wave: [ray 0's list, then the scatter staging area | ray 1's list]
+  using L = WaveLds<INTERP, kWave * NG, BIN>;
+  constexpr int kList1 = kWave * NG * 4;
+  __shared__ __align__(16) unsigned char s_mem[kWavesPerBlock][L::kBytes + kList1];
+  // nearest, RUN: the workgroup's cell sums, used when its rays are neighbours
+  constexpr bool kSums = RUN && INTERP == PXL_INTERP_NEAREST;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int64_t ray0 = P.ray_offset + 2 * ((int64_t)blockIdx.x * kWavesPerBlock + wave);
+  BinCursor cur{};
+  if constexpr (kSums) {
+    cur.sums = is_bundle(P);  // the same for every wave
+    if (cur.sums) {
+      for (uint32_t i = threadIdx.x; i < kSumSlots; i += kBlock) sum_keys()[i] = kSumEmpty;
+      for (uint32_t i = threadIdx.x; i < kSumSlots * 4; i += kBlock) sum_vals()[i] = 0.0;
+      __syncthreads();
+    }
+  }
+  if (ray0 < P.n_rays) train_pair<DT, INTERP, NG, BIN, RUN>(P, LP, ray0, lane, s_mem[wave], out, grad, B, cur);
+  if constexpr (kSums) {
+    if (!cur.sums) return;
+    __syncthreads();  // no wave has left: the decision is the workgroup's
+    for (uint32_t i = threadIdx.x; i < kSumSlots * 4; i += kBlock) {
+      const float v = (float)sum_vals()[i];
+      if (v != 0.f) atomic_add_f32(grad + (size_t)sum_keys()[i >> 2] * 4u + (i & 3u), v);
+    }
+  }
 }
 
 // Forward of two rays per wavefront for S <= 64 * NG: both rays classified together (up to two
@@ -1456,11 +1508,11 @@ template <int DT, int INTERP, bool BIN>
 void launch_train(const pxl::KParams& Q, const pxl::LossParams& LP, unsigned nb, float* out, float* grad,
                          const pxl::Bins& B, hipStream_t s) {
   const int S = Q.n_samples;
-  constexpr bool kRuns = INTERP == PXL_INTERP_TRILINEAR && !BIN;
+  constexpr bool kRuns = !BIN;
   const bool dense = kRuns && Q.occ == nullptr;
 #define PXL_LAUNCH_TRAIN(K) hipLaunchKernelGGL((K), dim3(nb), dim3(pxl::kBlock), 0, s, Q, LP, out, grad, B)
   if (S > 512) PXL_LAUNCH_TRAIN((pxl::k_train_long<DT, INTERP, BIN>));
-  else if (S > 256) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 8, BIN, kRuns>));
+  else if (S > 256) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 8, BIN, kRuns && INTERP == PXL_INTERP_TRILINEAR>));
   else if (S <= 64 && dense) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 1, BIN, kRuns>));
   else if (S <= 64) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 1, BIN, false>));
   else if (S <= 128 && dense) PXL_LAUNCH_TRAIN((pxl::k_train_pair<DT, INTERP, 2, BIN, kRuns>));

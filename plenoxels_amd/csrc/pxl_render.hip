@@ -326,7 +326,7 @@ __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP
       const int idx = (g << 6) + lane;
       const bool valid = idx < nk;
       const int k = valid ? list[idx] : 0;
-      if (valid) eval_kept<DT, INTERP>(P, R, k, V[g], CL[g]);
+      if (valid) eval_kept<DT, INTERP, BIN>(P, R, k, V[g], CL[g]);
       const float incl = wave_prefix_mul(1.f - V[g].w);
       const float Ti = T * wave_shift_up(incl, 1.f);
       bool proc = valid;
@@ -439,7 +439,7 @@ __device__ __forceinline__ void train_half_pair(const KParams& P, const LossPara
   const Ray R = select_ray(hi, R0, R1);
   float4 V = make_float4(0.f, 0.f, 0.f, 0.f);
   uint32_t CL = 0u;
-  if (valid) eval_kept<DT, INTERP>(P, R, k, V, CL);
+  if (valid) eval_kept<DT, INTERP, BIN>(P, R, k, V, CL);
   const float incl = half_prefix_mul(1.f - V.w);
   // lane 32 starts ray 1 with transmittance 1: the boundary value goes into the source lane
   // (31) before the shift, so every lane uses the DPP result.  (Selecting on the shifted value

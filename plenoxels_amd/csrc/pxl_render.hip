@@ -1156,7 +1156,10 @@ constexpr int64_t kMaxRaysPerLaunch = int64_t(1) << 26;  // at most 2^24 blocks 
 // samples kept) 128^3 cells, 4096 tiles: 44/50 at 2^18 samples, 80/64 at 2^19, 553/213 at 2^22;
 // 256^3, 32768 tiles: 505/525 at 2^22, 983/814 at 2^23; 48^3: 53/49 at 2^18, 193/113 at 2^20.
 // With a 5% occupancy (the host sees only that there is one): 128^3: 40/40 at 2^21, 73/56 at
-// 2^22; 256^3: 131/137 at 2^23; 48^3: 43/46 at 2^20, 132/87 at 2^22.
+// 2^22; 256^3: 131/137 at 2^23; 48^3: 43/46 at 2^20, 132/87 at 2^22.  Sparse scenes count a sample
+// by the cells it advances (delta / points distance, at most one): two neighbours in one cell share
+// their atomics' requests (110x78x80, three samples per cell, 5.9 M samples: 172/182 for forward
+// and backward).
 constexpr double kBinMinSamples = double(1 << 19), kBinTileSamples = 160.0;
 constexpr double kBinMinSamplesOcc = double(1 << 22), kBinTileSamplesOcc = 512.0;
 // Largest work buffer (a 512^3 training step of 2^19 rays x 512 samples asks for 11.1 GB; in
@@ -1304,8 +1307,12 @@ int for_ray_pieces(pxl::KParams P, int64_t rays_per_block, F&& fn, const char* w
 
 // Forward of two rays per wavefront (k_render_pair): where an occupancy leaves most rays at most
 // 32 samples.  Without one a ray keeps hundreds and the pair's rays run one after the other
-// (65537 rays x 192 samples, 110 kept: 318 us against k_render_fwd's 295).
-bool use_pairs(const pxl::KParams& P) { return P.occ != nullptr && P.n_samples <= 512; }
+// (65537 rays x 192 samples, 110 kept: 318 us against k_render_fwd's 295).  And from as many rays
+// on as fill the chip's 8192 wave slots in pairs: with fewer, half the waves take longer (100^3, 5%
+// occupied, 256 trilinear samples: 4000 rays 8.0 us in pairs and 6.8 one by one, 13000 12.7 and
+// 13.4, 40000 27.8 and 34.1).
+constexpr int64_t kPairRays = 1 << 14;
+bool use_pairs(const pxl::KParams& P) { return P.occ != nullptr && P.n_samples <= 512 && P.n_rays >= kPairRays; }
 
 template <int DT, int INTERP>
 void launch_fwd(const pxl::KParams& Q, unsigned nb, float* out, float* aux, hipStream_t s) {
@@ -1458,8 +1465,9 @@ int64_t pxl_scatter_work_bytes(const pxl_grid* grid, const pxl_march* march, int
   if (n_rays < 0) return fail(PXL_E_INVALID, "n_rays is negative");
   if (march->interp != PXL_INTERP_TRILINEAR || march->n_samples == 0) return 0;
   const BinPlan p = bin_plan(grid, march);
-  const double samples = (double)n_rays * march->n_samples;
   const bool occ = grid->occupancy != nullptr;
+  const double advance = occ ? std::min(1.0, std::fabs((double)march->delta) / march->pd) : 1.0;
+  const double samples = (double)n_rays * march->n_samples * advance;
   if (samples < (occ ? kBinMinSamplesOcc : kBinMinSamples) ||
       samples < p.tiles * (occ ? kBinTileSamplesOcc : kBinTileSamples))
     return 0;

@@ -151,10 +151,16 @@ class CameraRays:
                 raise ValueError("imgs and c2w must cover the same cameras")
 
 
+BIN_MIN_SAMPLES = 1 << 19  # below this many placed samples pxl_scatter_work_bytes is 0
+
+
 def _scatter_work(g, m, n_rays, device):
     """The tile-bin work buffer of a scatter (pxl_scatter_work_bytes), or None where float atomics
     are used: bins that would not pay, or a device without room for them (a quarter of the full
     size also does, in more pieces)."""
+    # never for nearest lookup and small batches: one call less where the host is what bounds a step
+    if m.interp == _lib.INTERP_NEAREST or n_rays * m.n_samples < BIN_MIN_SAMPLES:
+        return None
     n = _lib.lib().pxl_scatter_work_bytes(ctypes.byref(g), ctypes.byref(m), n_rays)
     if n < 0:
         _lib.check(int(n))

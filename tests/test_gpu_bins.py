@@ -11,7 +11,7 @@ import torch
 
 from oracle import plain
 from plenoxels_amd import MarchConfig, _lib, occupancy_dilate, pack_occupancy
-from plenoxels_amd.render import _grid_struct, _rays_struct, render_rays
+from plenoxels_amd.render import BIN_MIN_SAMPLES, _grid_struct, _rays_struct, render_rays
 from util import grad_close, say
 
 DEV = torch.device("cuda:0")
@@ -138,10 +138,13 @@ def test_scatter_work_bytes_rule():
     tri, near = (MarchConfig(128, 0.1, (0.0, 0.0, 0.0), 0.1, i).to_struct() for i in ("trilinear", "nearest"))
     q = lambda m, n: L.pxl_scatter_work_bytes(ctypes.byref(g), ctypes.byref(m), n)  # noqa: E731
     assert q(near, 1 << 20) == 0 and q(tri, 0) == 0 and q(tri, 100) == 0
+    assert q(tri, (BIN_MIN_SAMPLES - 1) // 128) == 0 and q(tri, BIN_MIN_SAMPLES // 128) > 0
     assert 0 < q(tri, 1 << 14) < q(tri, 1 << 15) <= q(tri, 1 << 26) <= 12 << 30
     assert q(tri, -1) == _lib.PXL_E_INVALID
     g.occupancy = 0x1000
     assert q(tri, 1 << 14) == 0 and q(tri, 1 << 15) > 0
+    fine = MarchConfig(128, 0.02, (0.0, 0.0, 0.0), 0.1, "trilinear").to_struct()  # five samples per cell
+    assert q(fine, 1 << 17) == 0 and q(fine, 1 << 18) > 0
     g.dims[0] = 1 << 18
     assert q(tri, 1 << 14) == 0
     assert L.pxl_scatter_work_bytes(None, ctypes.byref(tri), 5) == _lib.PXL_E_INVALID

@@ -14,11 +14,11 @@ DEV = torch.device("cuda:0")
 
 @pytest.mark.parametrize("Z", [1, 2, 3, 8, 33])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("occupied", [False, True])  # one ray per wave, two rays per wave
+@pytest.mark.parametrize("occupied", [False, True])  # one ray per wave; with 2^14 rays or more, two
 def test_half_gather_equals_float32(Z, dtype, occupied):
     say("half gather", Z, dtype, occupied)
     g = torch.Generator().manual_seed(Z)
-    dims, pd, R, S = (5, 6, Z), 0.5, 257, 70
+    dims, pd, R, S = (5, 6, Z), 0.5, (1 << 14) + 1 if occupied else 257, 70
     grid = (torch.rand(*dims, 4, generator=g) * 1.2 - 0.1).to(dtype)
     size = torch.tensor(dims) * pd
     a, b = (torch.rand(R, 3, generator=g) * size * 1.2 - 0.1 * size for _ in range(2))

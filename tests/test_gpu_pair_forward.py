@@ -1,4 +1,4 @@
-"""The two-rays-per-wavefront forward (occupancy given, up to 512 samples per ray) against the
+"""The two-rays-per-wavefront forward (occupancy given, up to 512 samples per ray, at least 2^14 rays) against the
 one-ray kernel: the same bits, outputs and saved state, for every chunk count, odd batches, rays
 with at most and with more than 32 kept samples, and early termination.  Without occupancy the
 one-ray kernel runs, so an occupancy of ones compares the two."""
@@ -39,13 +39,13 @@ def _forward(grid, o, d, cfg, bits):
 @pytest.mark.parametrize("dims", [(20, 20, 20), (70, 33, 40)])  # ~17 and ~40 samples per ray inside
 def test_pair_forward_equals_one_ray_forward(S, interp, t_stop, dtype, dims):
     say("pair forward", S, interp, t_stop, dtype, dims)
-    R = 131
+    R = (1 << 14) + 3
     grid, o, d, gmin, pd, delta, _ = _scene(dims, R, S, 7)
     grid = grid.to(dtype).to(DEV)
     o[-1], d[-1] = o[0] + 100.0, d[0]  # a ray that misses
     ones = pack_occupancy(torch.ones(dims, dtype=torch.bool, device=DEV))
     cfg = MarchConfig(S, delta, gmin, pd, interp, 0.0, t_stop)
-    for n in (R, R - 1, 1):
+    for n in (R, R - 1, 131):
         a, ax = _forward(grid, o[:n].contiguous().to(DEV), d[:n].contiguous().to(DEV), cfg, None)
         b, bx = _forward(grid, o[:n].contiguous().to(DEV), d[:n].contiguous().to(DEV), cfg, ones)
         assert torch.equal(a, b) and torch.equal(ax, bx)

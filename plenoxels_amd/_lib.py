@@ -222,6 +222,9 @@ def ptr(t):
 
 def stream_handle(device=None):
     """hipStream_t of torch's current stream on `device`."""
+    index = getattr(device, "index", None)
+    if index is not None and device.type == "cuda":  # a twentieth of the Stream object's time
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(index))
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 

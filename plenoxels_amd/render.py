@@ -44,13 +44,15 @@ class MarchConfig:
         if self.div_mode not in ("reciprocal", "divide"):
             raise ValueError(f"div_mode must be 'reciprocal' or 'divide', got {self.div_mode!r}")
         m.flags = _lib.FLAG_EXACT_DIV if self.div_mode == "divide" else 0
-        m.delta = float(np.float32(self.delta_step))
-        m.near = float(np.float32(self.near))
-        m.t_stop = float(self.t_stop)
-        m.pd = float(np.float32(self.points_distance))
-        m.inv_pd = float(np.float32(1.0) / np.float32(self.points_distance))
-        for a in range(3):
-            m.grid_min[a] = float(self.grid_min[a])
+        # a c_float field rounds a Python float to float32; the reciprocal is float32's own division
+        # (a double quotient of two floats rounds to the same float32)
+        m.delta = self.delta_step
+        m.near = self.near
+        m.t_stop = self.t_stop
+        m.pd = self.points_distance
+        m.inv_pd = 1.0 / m.pd if m.pd else float("inf")
+        gm = self.grid_min
+        m.grid_min[:] = (float(gm[0]), float(gm[1]), float(gm[2]))
         return m
 
 
@@ -73,8 +75,7 @@ def _grid_struct(grid, occupancy=None):
         raise ValueError("grid must be contiguous")
     g = _lib.Grid()
     g.data = grid.data_ptr()
-    for a in range(3):
-        g.dims[a] = grid.shape[a]
+    g.dims[:] = grid.shape[:3]
     g.channels = 4
     g.dtype = _DTYPES[grid.dtype]
     if occupancy is not None:

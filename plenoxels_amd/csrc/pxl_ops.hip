@@ -472,7 +472,15 @@ __global__ __launch_bounds__(256) void k_box_mean_rows(const float4* __restrict_
   const int per = kRowLdsCells / n;  // rows per batch (n <= kRowLdsCells)
   for (int64_t r0 = (int64_t)blockIdx.x * per; r0 < rows; r0 += (int64_t)gridDim.x * per) {
     const int nr = (int)min((int64_t)per, rows - r0);
-    for (int i = threadIdx.x; i < nr * n; i += blockDim.x) s_row[i] = in[r0 * n + i];
+    // all of a thread's loads in flight before the first is stored (256^3, k 25: 95 -> 83 us)
+    float4 v[kRowLdsCells / 256];
+#pragma unroll
+    for (int q = 0; q < kRowLdsCells / 256; ++q) {
+      const int i = q * 256 + (int)threadIdx.x;
+      v[q] = i < nr * n ? in[r0 * n + i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int q = 0; q < kRowLdsCells / 256; ++q) s_row[q * 256 + (int)threadIdx.x] = v[q];
     __syncthreads();
     for (int t = threadIdx.x; t < nr * n_out; t += blockDim.x) {
       const int rr = t / n_out, o = t - rr * n_out;

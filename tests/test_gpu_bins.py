@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import plain
-from plenoxels_amd import MarchConfig, _lib, occupancy_dilate, pack_occupancy
+from plenoxels_amd import MarchConfig, _lib, occupancy_dilate, pack_occupancy, train_step
 from plenoxels_amd.render import BIN_MIN_SAMPLES, _grid_struct, _rays_struct, render_rays
 from util import grad_close, say
 
@@ -148,3 +148,36 @@ def test_scatter_work_bytes_rule():
     g.dims[0] = 1 << 18
     assert q(tri, 1 << 14) == 0
     assert L.pxl_scatter_work_bytes(None, ctypes.byref(tri), 5) == _lib.PXL_E_INVALID
+
+
+@pytest.mark.gpu
+def test_binned_train_step_in_a_graph():
+    """A captured step (zero, tile-binned scatter) replayed several times, with eager work and new ray
+    directions between the replays, against the eager step on the same inputs."""
+    S, R = 128, 1 << 13
+    say("bins in a graph")
+    grid, o, d, gmin, pd, delta, tgt = _scene((32, 32, 32), R, S, 9)
+    grid, o, d, tgt = (t.to(DEV) for t in (grid, o, d, tgt))
+    cfg = MarchConfig(S, delta, gmin, pd, "trilinear")
+    grad, eager = torch.zeros_like(grid), torch.zeros_like(grid)
+
+    def step(out):
+        out.zero_()
+        train_step(grid, out, cfg=cfg, origins=o, dirs=d, targets=tgt)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(grad)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step(grad)
+    for i in range(4):
+        d.copy_(torch.nn.functional.normalize(d + 0.01 * i, dim=1))
+        step(eager)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        ok, info = grad_close(grad.cpu(), eager.cpu(), rel=1e-5)
+        assert ok and eager.abs().max() > 0, (i, info)

@@ -419,6 +419,16 @@ def beta_term_zero():
     return float(np.log(np.float32(BETA_EPS)) - np.log(np.float32(1.0 + BETA_EPS)))
 
 
+def _check_ray_values(name, v, device):
+    if v.dtype != torch.float32 or v.dim() != 1 or not v.is_contiguous() or v.device != device:
+        raise ValueError(f"{name} must be a contiguous 1-D float32 tensor on the work buffer's device")
+
+
+def _check_f64_scalar(name, t, device):
+    if t.dtype != torch.float64 or t.numel() != 1 or t.device != device:
+        raise ValueError(f"{name} must be a one-element float64 tensor on {device}")
+
+
 class LossMean:
     """mse_loss's mean (scripts/train.py:156) from per-ray squared errors (train_step's
     ray_sq_err) on the device: scale * sum in FP64, one launch, the same bits on every call
@@ -431,8 +441,7 @@ class LossMean:
     def __call__(self, ray_sq_err, n_rays=None):
         """0-dim float32 tensor: sum(ray_sq_err) / (4 * n_rays) (n_rays defaults to its length)."""
         v = ray_sq_err
-        if v.dtype != torch.float32 or v.dim() != 1 or not v.is_contiguous() or v.device != self.work.device:
-            raise ValueError("ray_sq_err must be a contiguous 1-D float32 tensor on the work buffer's device")
+        _check_ray_values("ray_sq_err", v, self.work.device)
         n_rays = v.shape[0] if n_rays is None else int(n_rays)
         if n_rays <= 0:
             raise ValueError("n_rays must be positive")
@@ -454,7 +463,17 @@ class LossTerms:
         """float32 (4,): mean squared error, tv_weight * TV, beta term (0 where not given), sum."""
         if n_rays <= 0:
             raise ValueError("n_rays must be positive")
-        out = torch.empty(4, dtype=torch.float32, device=self.work.device)
+        dev = self.work.device
+        _check_ray_values("ray_sq_err", ray_sq_err, dev)
+        if ray_beta is not None:
+            _check_ray_values("ray_beta", ray_beta, dev)
+            if ray_beta.shape != ray_sq_err.shape:
+                raise ValueError("ray_beta must have ray_sq_err's length")
+        if tv_sumsq is not None:
+            _check_f64_scalar("tv_sumsq", tv_sumsq, dev)
+        if dev.type != "cuda":
+            raise ValueError("the loss values are formed on a HIP device")
+        out = torch.empty(4, dtype=torch.float32, device=dev)
         _lib.check(_lib.lib().pxl_loss_terms(
             _lib.ptr(ray_sq_err), _lib.ptr(ray_beta), _lib.ptr(tv_sumsq), ray_sq_err.shape[0], 1.0 / (4.0 * n_rays),
             float(tv_weight), float(beta), n_samples * beta_term_zero(), float(n_samples), _lib.ptr(out),

@@ -76,8 +76,18 @@ def adam_pooled_step_(param, grad_out, k, stride, exp_avg, exp_avg_sq, step, *, 
     with it, in one pass over the grid (pxl_adam_pooled_step): the same bits, and the full
     gradient is never written."""
     X, Y, Z = (int(v) for v in param.shape[:3])
-    go = grad_out.float().contiguous()
     ws = _pool_workspace((X, Y, Z), k, stride, param.device)
+    pooled = tuple((n - k) // stride + 1 for n in (X, Y, Z)) + (4,)
+    if tuple(grad_out.shape) != pooled or grad_out.device != param.device:
+        raise ValueError(f"grad_out must have the pooled grid's shape {pooled} on {param.device}")
+    for name, t in (("param", param), ("exp_avg", exp_avg), ("exp_avg_sq", exp_avg_sq), ("grad_abs", grad_abs)):
+        if t is not None and (t.dtype != torch.float32 or tuple(t.shape) != (X, Y, Z, 4) or not t.is_contiguous()
+                              or t.device != param.device):
+            raise ValueError(f"{name} must be a contiguous ({X},{Y},{Z},4) float32 tensor on {param.device}")
+    if half_out is not None and (half_out.shape != param.shape or not half_out.is_contiguous()
+                                 or half_out.device != param.device):
+        raise ValueError("half_out must be contiguous with param's shape and device")
+    go = grad_out.float().contiguous()
     _lib.check(_lib.lib().pxl_adam_pooled_step(
         _lib.ptr(param), _lib.ptr(go), _lib.ptr(exp_avg), _lib.ptr(exp_avg_sq), _lib.ptr(grad_abs), X, Y, Z, int(k),
         int(stride), float(lr), float(betas[0]), float(betas[1]), float(eps), int(step), _lib.ptr(half_out),

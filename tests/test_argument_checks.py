@@ -3,6 +3,7 @@ range, or as another type, is refused before any pointer leaves Python."""
 import pytest
 import torch
 
+from plenoxels_amd.optim import adam_pooled_step_
 from plenoxels_amd.render import LossTerms
 
 
@@ -22,3 +23,23 @@ def test_loss_terms_rejects_what_its_kernel_would_misread():
             terms(sq, 64, tv_sumsq=bad, tv_weight=1.0)
     with pytest.raises(ValueError, match="HIP device"):
         terms(sq, 64, tv_sumsq=tv, tv_weight=1.0, ray_beta=bs, beta=1.0, n_samples=64)
+
+
+def test_adam_pooled_step_rejects_arrays_of_other_shapes():
+    dims, k, s = (8, 9, 10), 3, 2
+    p, m, v, a = (torch.zeros(*dims, 4) for _ in range(4))
+    go = torch.zeros(3, 4, 4, 4)
+    for bad in (go[:2], go[:, :3], torch.zeros(4, 4, 3, 4), torch.zeros(3, 4, 4), go.to("meta")):
+        with pytest.raises(ValueError, match="grad_out must"):
+            adam_pooled_step_(p, bad, k, s, m, v, 1, lr=1.0, grad_abs=a)
+    for bad in (m[:7], m.double(), torch.zeros(8, 9, 20, 4)[:, :, ::2], m.to("meta")):
+        with pytest.raises(ValueError, match="exp_avg must"):
+            adam_pooled_step_(p, go, k, s, bad, v, 1, lr=1.0)
+        with pytest.raises(ValueError, match="exp_avg_sq must"):
+            adam_pooled_step_(p, go, k, s, m, bad, 1, lr=1.0)
+        with pytest.raises(ValueError, match="grad_abs must"):
+            adam_pooled_step_(p, go, k, s, m, v, 1, lr=1.0, grad_abs=bad)
+    with pytest.raises(ValueError, match="half_out must"):
+        adam_pooled_step_(p, go, k, s, m, v, 1, lr=1.0, half_out=torch.zeros(7, 9, 10, 4, dtype=torch.bfloat16))
+    with pytest.raises(ValueError, match="average pooling needs"):
+        adam_pooled_step_(p, go, 9, s, m, v, 1, lr=1.0)

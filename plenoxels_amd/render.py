@@ -531,6 +531,8 @@ def alpha_occupancy(grid, interp="nearest", tv_sumsq=None):
     changes no finite result of the render and training kernels: their clamped alpha is 0 and
     the clamp's gradient mask is 0.  tv_sumsq (float32 grids): a float64 device scalar to which
     the same read of the grid adds optim.tv_sumsq's sum."""
+    if tv_sumsq is not None:
+        _check_f64_scalar("tv_sumsq", tv_sumsq, grid.device)
     X, Y, Z = (int(v) for v in grid.shape[:3])
     bits = torch.empty(occupancy_words((X, Y, Z)), dtype=torch.int32, device=grid.device)
     g = _grid_struct(grid, None)

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from plenoxels_amd.optim import adam_pooled_step_
-from plenoxels_amd.render import LossTerms
+from plenoxels_amd.render import LossTerms, alpha_occupancy
 
 
 def test_loss_terms_rejects_what_its_kernel_would_misread():
@@ -43,3 +43,11 @@ def test_adam_pooled_step_rejects_arrays_of_other_shapes():
         adam_pooled_step_(p, go, k, s, m, v, 1, lr=1.0, half_out=torch.zeros(7, 9, 10, 4, dtype=torch.bfloat16))
     with pytest.raises(ValueError, match="average pooling needs"):
         adam_pooled_step_(p, go, 9, s, m, v, 1, lr=1.0)
+
+
+def test_alpha_occupancy_rejects_a_tv_sum_of_another_type_or_place():
+    grid = torch.zeros(4, 4, 4, 4)
+    for bad in (torch.zeros(1), torch.zeros(2, dtype=torch.float64), torch.zeros(0, dtype=torch.float64),
+                torch.zeros(1, dtype=torch.float64, device="meta")):
+        with pytest.raises(ValueError, match="tv_sumsq must be"):
+            alpha_occupancy(grid, "nearest", tv_sumsq=bad)

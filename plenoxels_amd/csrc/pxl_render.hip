@@ -1148,7 +1148,8 @@ using pxl_host::occupancy_words;
 using pxl_host::launched;
 using pxl_host::stride_blocks;
 
-constexpr int64_t kMaxRaysPerLaunch = int64_t(1) << 26;  // at most 2^24 blocks per launch
+// A launch holds fewer than 2^32 threads: at most 2^23 blocks of 256 (one ray per wavefront).
+constexpr int64_t kMaxRaysPerLaunch = int64_t(1) << 25;
 
 // Tile bins (pxl_scatter_work_bytes): where they pay, by placed samples.  Their cost grows with
 // the tiles that are reached (each flushes up to ~240 requests), the corner atomics' with the kept
@@ -1387,7 +1388,7 @@ BinPlan bin_plan(const pxl_grid* grid, const pxl_march* march) {
 int64_t bin_rays(const BinPlan& p, int64_t S, int64_t work_bytes) {
   int64_t n = work_bytes > p.fixed ? (work_bytes - p.fixed) / p.per_ray : 0;
   n = std::min(n, (int64_t(1) << 31) / std::max<int64_t>(S, 1));  // 32-bit slots
-  return n & ~int64_t(1);
+  return std::min(n, kMaxRaysPerLaunch) & ~int64_t(1);
 }
 
 pxl::Bins bin_layout(const BinPlan& p, int64_t S, int64_t n, int64_t rays_per_region, void* work) {
@@ -1471,7 +1472,8 @@ int64_t pxl_scatter_work_bytes(const pxl_grid* grid, const pxl_march* march, int
   if (samples < (occ ? kBinMinSamplesOcc : kBinMinSamples) ||
       samples < p.tiles * (occ ? kBinTileSamplesOcc : kBinTileSamples))
     return 0;
-  const int64_t most = std::max<int64_t>(2, (kBinMaxBytes - p.fixed) / p.per_ray) & ~int64_t(1);
+  const int64_t fit = std::max<int64_t>(2, (kBinMaxBytes - p.fixed) / p.per_ray) & ~int64_t(1);
+  const int64_t most = std::min(fit, kMaxRaysPerLaunch);
   return p.fixed + p.per_ray * std::min<int64_t>(most, (n_rays + 1) & ~int64_t(1));
 }
 

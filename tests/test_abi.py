@@ -266,6 +266,17 @@ def test_corner_block_validation_before_any_hip_call():
     assert L.pxl_alpha_occupancy(None, 1, ctypes.c_void_p(0x10), None) == _lib.PXL_E_INVALID
 
 
+def test_scatter_work_bytes_stay_within_one_launch():
+    """A piece of a binned scatter is one launch of a wavefront per ray, below 2^32 threads: no buffer
+    is sized for more rays, however few bytes each needs."""
+    L = _lib.lib()
+    g, m, _ = _valid()
+    m.interp, m.n_samples = _lib.INTERP_TRILINEAR, 1
+    q = lambda n: L.pxl_scatter_work_bytes(ctypes.byref(g), ctypes.byref(m), n)  # noqa: E731
+    assert 0 < q(1 << 24) < q((1 << 24) + 2) < q(1 << 25)
+    assert q(1 << 25) == q(1 << 26) == q(1 << 40) < 12 << 30
+
+
 def test_scaled_sum_validation():
     L = _lib.lib()
     assert L.pxl_scaled_sum_work_bytes() == 1024

@@ -109,6 +109,46 @@ def test_render_rays_backward_above_the_bin_threshold(S, interp):
 
 
 @pytest.mark.gpu
+def test_more_rays_than_one_launch():
+    """2^26 + 5 rays of one and two samples: more than one launch takes, forward, backward and train step,
+    binned (whose pieces the work buffer's bytes alone would not bound) and direct."""
+    R, dims, pd = (1 << 26) + 5, (24, 25, 26), 0.1
+    g = torch.Generator(device=DEV).manual_seed(8)
+    grid = torch.rand(*dims, 4, device=DEV, generator=g) * 0.5
+    o = torch.rand(R, 3, device=DEV, generator=g) * 2.2
+    d = torch.zeros(R, 3, device=DEV)
+    d[:, 2] = 1.0
+    up = torch.rand(R, 4, device=DEV, generator=g)
+    tgt = -up  # every sample's gradient is positive, so that no cell's sum cancels
+    for S in (1, 2):
+        say("more rays than one launch", S)
+        cfg = MarchConfig(S, 0.11, (0.0, 0.0, 0.0), pd, "trilinear")
+        kw = dict(num_samples=S, delta_step=0.11, grid_min=(0.0, 0.0, 0.0), points_distance=pd, interp="trilinear")
+        leaf = grid.clone().requires_grad_(True)
+        g_, m = _grid_struct(grid, None), cfg.to_struct()
+        assert _lib.lib().pxl_scatter_work_bytes(ctypes.byref(g_), ctypes.byref(m), R) > 0
+        out = render_rays(leaf, o, d, **kw)
+        out.backward(up)
+        parts = grid.clone().requires_grad_(True)
+        for a in range(0, R, 1 << 23):
+            w = render_rays(parts, o[a:a + (1 << 23)], d[a:a + (1 << 23)], **kw)
+            assert torch.equal(w, out[a:a + (1 << 23)])
+            w.backward(up[a:a + (1 << 23)])
+        # a cell's ~10^4 records arrive in a few thousand FP32 additions of positive terms, in another
+        # order: each rounds to 2^-24, sqrt(5000) * 2^-24 = 4e-6 typically and 3e-4 if all round alike
+        ok, info = grad_close(leaf.grad.cpu(), parts.grad.cpu())
+        assert ok, info
+        grads = []
+        for n in (R, R // 2):
+            grad = torch.zeros_like(grid)
+            for a in range(0, R, n):
+                train_step(grid, grad, cfg=cfg, origins=o[a:a + n], dirs=d[a:a + n], targets=tgt[a:a + n], n_total_rays=R)
+            grads.append(grad.cpu())
+        ok, info = grad_close(grads[0], grads[1])
+        assert ok, info
+
+
+@pytest.mark.gpu
 def test_binned_integer_coordinates():
     """Samples at exact integer coordinates (ceil == floor) and on the last cell, whose ceil is itself."""
     X, pd = 16, 0.25

@@ -1421,7 +1421,8 @@ int for_bin_pieces(const pxl_grid* grid, const pxl_march* march, pxl::KParams P,
                           int64_t rays_per_region, void* work, int64_t work_bytes, float* grad_grid, hipStream_t s,
                           F&& fn, const char* what) {
   const BinPlan plan = bin_plan(grid, march);
-  const int64_t per = std::min(bin_rays(plan, march->n_samples, work_bytes), (P.n_rays + 1) & ~int64_t(1));
+  // bin_rays is even
+  const int64_t per = (std::min(bin_rays(plan, march->n_samples, work_bytes), P.n_rays) + 1) & ~int64_t(1);
   const pxl::Bins B = bin_layout(plan, march->n_samples, per, rays_per_region, work);
   const int64_t total = P.n_rays;
   const int64_t zero4 = (4 + plan.tiles + 3) / 4;  // the layout rounds this up to whole float4s
@@ -1474,7 +1475,7 @@ int64_t pxl_scatter_work_bytes(const pxl_grid* grid, const pxl_march* march, int
     return 0;
   const int64_t fit = std::max<int64_t>(2, (kBinMaxBytes - p.fixed) / p.per_ray) & ~int64_t(1);
   const int64_t most = std::min(fit, kMaxRaysPerLaunch);
-  return p.fixed + p.per_ray * std::min<int64_t>(most, (n_rays + 1) & ~int64_t(1));
+  return p.fixed + p.per_ray * ((std::min(most, n_rays) + 1) & ~int64_t(1));  // most is even
 }
 
 int pxl_render_bwd(const pxl_grid* grid, const pxl_march* march, const pxl_rays* rays,

@@ -275,6 +275,9 @@ def test_scatter_work_bytes_stay_within_one_launch():
     q = lambda n: L.pxl_scatter_work_bytes(ctypes.byref(g), ctypes.byref(m), n)  # noqa: E731
     assert 0 < q(1 << 24) < q((1 << 24) + 2) < q(1 << 25)
     assert q(1 << 25) == q(1 << 26) == q(1 << 40) < 12 << 30
+    # counts next to the type's limit are rounded up to a pair after the bound, not before
+    assert q(2 ** 63 - 1) == q(2 ** 63 - 2) == q(1 << 25)
+    assert q((1 << 24) + 1) == q((1 << 24) + 2)
 
 
 def test_scaled_sum_validation():

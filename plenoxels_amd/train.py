@@ -20,7 +20,7 @@ import torch
 
 from . import _lib
 from .checkpoint import save_grid
-from .grid_functions import average_pool3d_grid
+from .grid_functions import average_pool3d_grid, pool_backward_
 from .optim import adam_pooled_step_, adam_step_, adam_tv_step_, tv_backward_, tv_sumsq
 from .render import (CameraRays, CornerBlockPair, LossTerms, MarchConfig, alpha_occupancy, blocks_reduce, fill_,
                      train_step)
@@ -104,8 +104,9 @@ class Trainer:
         self.grid = torch.zeros((X, Y, Z, 4), dtype=torch.float32, device=self.dev)
         if init_grid is not None:  # the reference starts from zeros (src/grid_functions.py:214)
             self.grid.copy_(init_grid)
-        self.grad = torch.zeros_like(self.grid)
-        self._grad_zero = True  # self.grad is all zero (the fused TV + Adam pass can leave it so)
+        self._grad = torch.zeros_like(self.grid)
+        self._grad_zero = True  # self._grad is all zero (the fused TV + Adam pass can leave it so)
+        self._pooled_grad = None  # (pooled gradient, k, stride) of the last step, if it was a pooled one
         self.exp_avg = torch.zeros_like(self.grid)
         self.exp_avg_sq = torch.zeros_like(self.grid)
         self.grad_abs = torch.zeros_like(self.grid)
@@ -128,6 +129,17 @@ class Trainer:
             ls = torch.linspace(0, end=1, steps=m, device=self.dev)
             self.even_uv = torch.cartesian_prod(ls, ls).repeat([self.B, 1, 1])
 
+    @property
+    def grad(self):
+        """The full grid's gradient buffer, as the last step left it.  A pooled step's Adam pass forms
+        the full gradient in registers; a caller that asks for it gets it from the pooled one, the
+        same bits."""
+        if self._pooled_grad is not None:
+            (go, k, stride), self._pooled_grad = self._pooled_grad, None
+            pool_backward_(go, self.dims, k, stride, self._grad, accumulate=False)
+            self._grad_zero = False
+        return self._grad
+
     def _uniforms(self, i):
         if self.uniforms_fn is not None:
             return self.uniforms_fn(i).to(self.dev).float()
@@ -147,9 +159,9 @@ class Trainer:
 
     def step(self, i):
         """One training step; returns device scalars {"closs", "tvloss", "betaloss", "loss"}."""
-        X, Y, Z = self.dims
         k = receptive_field(i)
         pooled = k > 1 and self.progressive
+        self._pooled_grad = None
         if pooled:
             stride = max(1, k // 4)
             start = int(k / 2)
@@ -167,7 +179,7 @@ class Trainer:
             gmin = tuple(grid_coordinate(0, s, self.pd) for s in self.dims)
             pd = self.pd
             grid = self.grid if self.render_copy is None else self.render_copy
-            grad = self.grad
+            grad = self._grad
             if not self.use_blocks and not self._grad_zero:
                 fill_(grad, 0.0)
             self._grad_zero = False
@@ -220,20 +232,21 @@ class Trainer:
         if use_beta:
             out["betaloss"] = terms[2]
         self.step_count += 1
-        if pooled:  # the pooling backward is part of the Adam pass: self.grad is neither read nor written
-            adam_pooled_step_(self.grid, grad, k, max(1, k // 4), self.exp_avg, self.exp_avg_sq, self.step_count,
+        if pooled:  # the pooling backward is part of the Adam pass: self._grad is neither read nor written
+            adam_pooled_step_(self.grid, grad, k, stride, self.exp_avg, self.exp_avg_sq, self.step_count,
                               lr=self.lr, grad_abs=self.grad_abs, half_out=self.render_copy)
+            self._pooled_grad = (grad, k, stride)
         elif fused_tv:
             if self._grid_next is None:
                 self._grid_next = torch.empty_like(self.grid)
             # the pass leaves the gradient zero for the next step (no separate zero-fill)
-            adam_tv_step_(self.grid, self._grid_next, self.grad, self.exp_avg, self.exp_avg_sq, self.step_count,
+            adam_tv_step_(self.grid, self._grid_next, self._grad, self.exp_avg, self.exp_avg_sq, self.step_count,
                           tv_sumsq=self.tvs, tv_weight=self.tv, lr=self.lr, grad_abs=self.grad_abs,
                           half_out=self.render_copy, zero_grad=True)
             self._grad_zero = True
             self.grid, self._grid_next = self._grid_next, self.grid
         else:
-            adam_step_(self.grid, self.grad, self.exp_avg, self.exp_avg_sq, self.step_count, lr=self.lr,
+            adam_step_(self.grid, self._grad, self.exp_avg, self.exp_avg_sq, self.step_count, lr=self.lr,
                        grad_abs=self.grad_abs, half_out=self.render_copy)
         out["loss"] = terms[3]
         return out

@@ -155,6 +155,26 @@ class CameraRays:
 BIN_MIN_SAMPLES = 1 << 19  # below this many placed samples pxl_scatter_work_bytes is 0
 
 
+# Buffers up to this size are taken without asking for room: the question is a driver call of ~6 us.
+WORK_UNASKED_BYTES = 256 << 20
+
+
+def _has_room(n, device):
+    """Whether torch's allocator can serve n bytes from the device's free memory or its own cache.
+    A request that cannot be met makes it give its whole cache back before it fails, and a step that
+    tried each time would pay for that each time."""
+    free, total = torch.cuda.mem_get_info(device)
+    fraction = torch.cuda.get_per_process_memory_fraction(device)
+    n += 2 << 20  # the allocator's rounding of large blocks
+    if fraction >= 1.0 and n <= free:
+        return True
+    if torch.cuda.is_current_stream_capturing():
+        return False  # a capture's pool does not share the cache, and must not make torch release it
+    reserved = torch.cuda.memory_reserved(device)
+    free = min(free, int(total * fraction) - reserved)
+    return n <= free + reserved - torch.cuda.memory_allocated(device)
+
+
 def _scatter_work(g, m, n_rays, device):
     """The tile-bin work buffer of a scatter (pxl_scatter_work_bytes), or None where float atomics
     are used: bins that would not pay, or a device without room for them (a quarter of the full
@@ -168,6 +188,8 @@ def _scatter_work(g, m, n_rays, device):
     if n == 0:
         return None
     for size in (n, n // 4):
+        if size > WORK_UNASKED_BYTES and not _has_room(size, device):
+            continue
         try:
             return torch.empty(size, dtype=torch.uint8, device=device)
         except torch.OutOfMemoryError:

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import plain
-from plenoxels_amd import MarchConfig, _lib, occupancy_dilate, pack_occupancy, train_step
+from plenoxels_amd import MarchConfig, _lib, occupancy_dilate, pack_occupancy, render, train_step
 from plenoxels_amd.render import BIN_MIN_SAMPLES, _grid_struct, _rays_struct, render_rays
 from util import grad_close, say
 
@@ -221,3 +221,13 @@ def test_binned_train_step_in_a_graph():
         torch.cuda.synchronize()
         ok, info = grad_close(grad.cpu(), eager.cpu(), rel=1e-5)
         assert ok and eager.abs().max() > 0, (i, info)
+
+
+@pytest.mark.gpu
+def test_binned_train_step_asks_for_room_in_a_graph(monkeypatch):
+    """The question for free memory, which only large work buffers ask, is allowed under capture."""
+    asked, has_room = [], render._has_room
+    monkeypatch.setattr(render, "WORK_UNASKED_BYTES", 0)
+    monkeypatch.setattr(render, "_has_room", lambda n, dev: asked.append(has_room(n, dev)) or asked[-1])
+    test_binned_train_step_in_a_graph()
+    assert len(asked) == 6 and all(asked)

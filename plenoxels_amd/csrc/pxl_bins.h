@@ -61,8 +61,16 @@ struct BinCursor {
 };
 
 // One group's kept samples as records slot + rank and runs.  Called by the whole wave.
+// Samples that no cell takes a gradient from get no record: all of a trained grid's empty space, where
+// alpha is below zero at every corner (open: not so; alpha's gradient is clipped, the colours' are zero).  256^3
+// cells, 90% of them empty, no occupancy, a train step of 2^24 samples: 966 -> 558 us (664 with corner
+// atomics, which skip zeros too); 64^3, 97% empty, 2^23 samples: 247 -> 80 (114).  Dense grids pay at
+// most 1%.  Whether the colours are clipped is not looked at: that takes 16 to 21 more registers.
+// A run goes on over dropped samples; the tiles of the kept ones are still monotone along a ray,
+// so bin_ray_runs' bound holds.
 __device__ __forceinline__ void emit_chunk(const KParams& P, const Bins& B, const Ray& R, int lane, int k, bool keep,
-                                           const float4& gv, BinCursor& cur) {
+                                           bool open, const float4& gv, BinCursor& cur) {
+  keep = keep && (gv.x != 0.f || gv.y != 0.f || gv.z != 0.f || (open && gv.w != 0.f));
   const uint64_t km = __ballot(keep);
   if (km == 0ull) return;
   float nx, ny, nz;
@@ -71,9 +79,9 @@ __device__ __forceinline__ void emit_chunk(const KParams& P, const Bins& B, cons
   if (keep)
     tile = (((uint32_t)floorf(nx) >> 3) * P.occ_ty + ((uint32_t)floorf(ny) >> 3)) * P.occ_tz +
            ((uint32_t)floorf(nz) >> 3);
-  const uint32_t prev =
-      (uint32_t)__builtin_amdgcn_update_dpp((int)0xfffffffeu, (int)tile, DPP_WAVE_SHR1, 0xf, 0xf, false);
-  const bool head = keep && tile != prev;  // a lane behind a dropped one starts a run too
+  const uint64_t below = km & ~(~0ull << lane);
+  const uint32_t prev = (uint32_t)__shfl((int)tile, below ? 63 - __builtin_clzll(below) : lane);
+  const bool head = keep && (below == 0ull || tile != prev);
   const uint64_t hm = __ballot(head);
   const uint32_t slot = cur.slot + (uint32_t)lane_rank(km);
   if (keep) {

@@ -549,8 +549,9 @@ __device__ __forceinline__ void load_corners(const KParams& P, const TriCell& t,
 // (sum of the eight corner weights (wx*wy)*wz times the corner; the reference's nested lerps
 // src/grid_functions.py:34-42 compute the same polynomial).  clip: bit c (nearest) or
 // 4j + c (trilinear corner j = 4*bx + 2*by + bz, b = 0 ceil / 1 floor, the corner order of
-// src/grid_functions.py:238-243).
-template <int DT, int INTERP, bool ZPAIR = true>
+// src/grid_functions.py:238-243).  OPEN (trilinear):
+// clip is instead whether some corner's raw alpha is at least zero.
+template <int DT, int INTERP, bool ZPAIR = true, bool OPEN = false>
 __device__ __forceinline__ void eval_kept(const KParams& P, const Ray& R, int k, float4& v,
                                           uint32_t& clip) {
   float nx, ny, nz;
@@ -571,15 +572,18 @@ __device__ __forceinline__ void eval_kept(const KParams& P, const Ray& R, int k,
     load_corners<DT, ZPAIR>(P, t, raw);
     const float ofx = 1.f - t.fx, ofy = 1.f - t.fy, ofz = 1.f - t.fz;
     v = make_float4(0.f, 0.f, 0.f, 0.f);
+    float top = -1.f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float w = ((j & 4 ? ofx : t.fx) * (j & 2 ? ofy : t.fy)) * (j & 1 ? ofz : t.fz);
       const float4 c = cell_value<DT>(raw[j]);
+      if constexpr (OPEN) top = fmaxf(top, c.w);
       v.x = fmaf(w, clip_ch(c.x, clip, 4 * j + 0), v.x);
       v.y = fmaf(w, clip_ch(c.y, clip, 4 * j + 1), v.y);
       v.z = fmaf(w, clip_ch(c.z, clip, 4 * j + 2), v.z);
       v.w = fmaf(w, clip_ch(c.w, clip, 4 * j + 3), v.w);
     }
+    if constexpr (OPEN) clip = top >= 0.f ? 1u : 0u;
   }
 }
 

@@ -152,7 +152,8 @@ __global__ __launch_bounds__(kBlock) void k_render_fwd(KParams P, float* __restr
 
 // One group of the reverse sweep: given the group's clipped values, transmittance and Qn
 // (the suffix value just behind the group), emit dL/dvalue per sample, scatter it, and
-// return in Qn the suffix value in front of the group.
+// return in Qn the suffix value in front of the group.  clip: eval_kept's mask; with
+// BIN, whether some corner's raw alpha is at least zero.
 template <int INTERP, bool RUNS, bool BIN>
 __device__ __forceinline__ void reverse_chunk(const KParams& P, const Ray& R, int lane, int k,
                                               bool keep, const float4& v, uint32_t clip,
@@ -185,7 +186,7 @@ __device__ __forceinline__ void reverse_chunk(const KParams& P, const Ray& R, in
     gv.w = Ti * (g.x * (v.x - s0) + g.y * (v.y - s1) + g.z * (v.z - s2) + g.w * (1.f - s3));
     if (beta_scale != 0.f) gv.w += beta_scale * beta_dloss(v.w);
   }
-  if constexpr (BIN) emit_chunk(P, B, R, lane, k, keep, gv, cur);
+  if constexpr (BIN) emit_chunk(P, B, R, lane, k, keep, clip != 0u, gv, cur);
   else scatter_chunk<INTERP, RUNS>(P, R, lane, k, keep, clip, gv, grad, s_cell, s_val, cur.sums);
   Qn = make_float4(readlane(f.a0, 0), readlane(f.a1, 0), readlane(f.a2, 0), readlane(f.a3, 0));
 }
@@ -238,7 +239,7 @@ __device__ __forceinline__ void reverse_sweep(const KParams& P, const Ray& R, in
     wave_lds_sync();
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     uint32_t clip = 0u;
-    if (valid) eval_kept<DT, INTERP>(P, R, k, v, clip);
+    if (valid) eval_kept<DT, INTERP, true, BIN>(P, R, k, v, clip);
     const float incl = wave_prefix_mul(1.f - v.w);
     const float Ti = T0 * wave_shift_up(incl, 1.f);
     if constexpr (BIN) cur.slot = slot0 + (uint32_t)(gi * kWave);
@@ -252,8 +253,10 @@ __device__ __forceinline__ BinCursor bin_cursor(const KParams& P, const Bins& B,
   return BinCursor{ray * (uint32_t)P.n_samples, ray / rays * B.run_cap, 0u, false};
 }
 
+// BIN: the registers of six waves per SIMD, eight with half storage (one or two too many without the
+// bound, and a wave fewer).
 template <int DT, int INTERP, bool BIN>
-__global__ __launch_bounds__(kBlock) void k_render_bwd(KParams P, const float* __restrict__ grad_out,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(!BIN ? 1 : DT == PXL_DTYPE_F32 ? 6 : 8))) void k_render_bwd(KParams P, const float* __restrict__ grad_out,
                                                         const float* __restrict__ aux,
                                                         float* __restrict__ grad, Bins B) {
   using L = WaveLds<INTERP, kWave, BIN>;
@@ -307,7 +310,7 @@ __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP
   const int S = P.n_samples;
   const int ng = (nk + 63) >> 6;
   float4 V[NG];
-  uint32_t CL[NG];
+  uint32_t CL[BIN ? 1 : NG];  // clip masks; BIN: a bit per group (emit_chunk's open)
   float TI[NG];
   int KI[NG];
   uint64_t KEEP[NG];
@@ -318,7 +321,7 @@ __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
     V[g] = make_float4(0.f, 0.f, 0.f, 0.f);
-    CL[g] = 0u;
+    if (!BIN || g == 0) CL[g] = 0u;
     TI[g] = 0.f;
     KI[g] = 0;
     KEEP[g] = 0ull;
@@ -326,7 +329,13 @@ __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP
       const int idx = (g << 6) + lane;
       const bool valid = idx < nk;
       const int k = valid ? list[idx] : 0;
-      if (valid) eval_kept<DT, INTERP, BIN>(P, R, k, V[g], CL[g]);
+      if constexpr (BIN) {
+        uint32_t open = 0u;
+        if (valid) eval_kept<DT, INTERP, true, true>(P, R, k, V[g], open);
+        CL[0] |= open << g;
+      } else {
+        if (valid) eval_kept<DT, INTERP, false>(P, R, k, V[g], CL[g]);
+      }
       const float incl = wave_prefix_mul(1.f - V[g].w);
       const float Ti = T * wave_shift_up(incl, 1.f);
       bool proc = valid;
@@ -361,8 +370,9 @@ __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP
     if (g < ng && KEEP[g] != 0ull) {
       const bool keep = (KEEP[g] >> lane) & 1ull;
       if constexpr (BIN) cur.slot = slot0 + (uint32_t)(g * kWave);
-      reverse_chunk<INTERP, RUN, BIN>(P, R, lane, KI[g], keep, V[g], CL[g], TI[g], gl, LP.beta_scale, Qn,
-                                                grad, s_cell, s_val, B, cur);
+      const uint32_t clip = BIN ? (CL[0] >> g) & 1u : CL[BIN ? 0 : g];
+      reverse_chunk<INTERP, RUN, BIN>(P, R, lane, KI[g], keep, V[g], clip, TI[g], gl, LP.beta_scale, Qn, grad, s_cell,
+                                      s_val, B, cur);
     }
   }
 }
@@ -439,7 +449,7 @@ __device__ __forceinline__ void train_half_pair(const KParams& P, const LossPara
   const Ray R = select_ray(hi, R0, R1);
   float4 V = make_float4(0.f, 0.f, 0.f, 0.f);
   uint32_t CL = 0u;
-  if (valid) eval_kept<DT, INTERP, BIN>(P, R, k, V, CL);
+  if (valid) eval_kept<DT, INTERP, BIN, BIN>(P, R, k, V, CL);
   const float incl = half_prefix_mul(1.f - V.w);
   // lane 32 starts ray 1 with transmittance 1: the boundary value goes into the source lane
   // (31) before the shift, so every lane uses the DPP result.  (Selecting on the shifted value
@@ -501,7 +511,7 @@ __device__ __forceinline__ void train_half_pair(const KParams& P, const LossPara
     gv.w = Ti * (gl.x * (V.x - s0) + gl.y * (V.y - s1) + gl.z * (V.z - s2) + gl.w * (1.f - s3));
     if (LP.beta_scale != 0.f) gv.w += LP.beta_scale * beta_dloss(V.w);
   }
-  if constexpr (BIN) emit_chunk(P, B, R, lane, k, proc, gv, cur);
+  if constexpr (BIN) emit_chunk(P, B, R, lane, k, proc, CL != 0u, gv, cur);
   else scatter_chunk<INTERP, RUN>(P, R, lane, k, proc, CL, gv, grad, s_cell, s_val, cur.sums);
 }
 

@@ -85,6 +85,35 @@ def test_binned_train_step_equals_direct(dims, R, S, dtype, occupied, t_stop):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dims,R,S,dtype", [
+    ((9, 17, 5), 130, 40, torch.float32),        # two rays share a group of 64 lanes
+    ((24, 24, 24), 501, 128, torch.bfloat16),
+    ((33, 10, 70), 257, 300, torch.float16),
+    ((24, 20, 28), 300, 700, torch.float32),     # one ray per wavefront
+])
+def test_samples_without_a_gradient_get_no_record(dims, R, S, dtype):
+    """A grid whose empty cells have alpha below zero: a sample with such cells at all corners is dropped,
+    within a run too, and the gradient stays; where every sample is such a one no item is left."""
+    say("bins, empty cells", dims, R, S, dtype)
+    grid, o, d, gmin, pd, delta, tgt = _scene(dims, R, S, 11)
+    g = torch.Generator().manual_seed(12)
+    grid[..., 3][torch.rand(dims, generator=g) < 0.8] = -0.02
+    grid[..., :3][torch.rand(*dims, 3, generator=g) < 0.4] = 1.5
+    o, d, tgt = o.to(DEV), d.to(DEV), tgt.to(DEV)
+    cfg = MarchConfig(S, delta, gmin, pd, "trilinear")
+    work = torch.empty(1 << 26, dtype=torch.uint8, device=DEV)
+    items = work[: 4].view(torch.int32)  # the buffer's first word counts the tile sums' items
+    a, b = (_train(grid.to(dtype).to(DEV), o, d, tgt, cfg, None, w) for w in (None, work))
+    assert int(items) > 0 and a[3].abs().max() > 0
+    ok, info = grad_close(b[3], a[3], rel=1e-5)
+    assert ok, info
+    empty = grid.clone()
+    empty[..., 3] = -0.5
+    _, _, _, grad = _train(empty.to(dtype).to(DEV), o, d, tgt, cfg, None, work)
+    assert int(items) == 0 and grad.abs().max() == 0
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("S,interp", [(96, "trilinear"), (700, "trilinear"), (96, "nearest")])
 def test_render_rays_backward_above_the_bin_threshold(S, interp):
     """Large enough a batch that render_rays' backward takes the bins (trilinear), against the plain

@@ -633,47 +633,99 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 
 // chunks in one round trip; above 128 samples a chunk of each at a time, as many as the sample count
 // needs -- all eight in flight took 114 registers and 328 us where the loop takes 229, an 600x600
 // view with 331 nearest samples) and k_train_pair's half-wave group when each ray keeps at most 32 samples, else
-// the rays' groups one after the other.  Every value is formed by the operation tree of
+// groups of one ray.  Every value is formed by the operation tree of
 // forward_sweep, so outputs and aux are the same bits.
 // 800x800 view of a 256^3 FP16 grid with ~5% occupancy, 256 trilinear samples: 663 us with
 // one ray per wave, 451 us with two.
-template <int DT, int INTERP, int NG>
-__device__ __forceinline__ void fwd_ray(const KParams& P, const Ray& R, int64_t ray, const int* list, int nk, int lane,
-                                        float* __restrict__ out, float* __restrict__ aux) {
-  float* ax = aux ? aux + ray * P.aux_stride : nullptr;
-  const int ng = (nk + 63) >> 6;
-  float T = 1.f, cr = 0.f, cg = 0.f, cb = 0.f, ca = 0.f;
-  int n_proc = P.n_samples, done = 0;
-  for (bool stop = false; done < ng && !stop; ++done) {
-    const int idx = (done << 6) + lane;
-    const bool valid = idx < nk;
-    const int k = valid ? list[idx] : 0;
-    if (ax && lane == 0) {
-      ax[2 + 2 * done] = T;
-      ax[3 + 2 * done] = __int_as_float(k);
-    }
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    uint32_t clip;
-    if (valid) eval_kept<DT, INTERP>(P, R, k, v, clip);
-    const float incl = wave_prefix_mul(1.f - v.w);
-    const float Ti = T * wave_shift_up(incl, 1.f);
-    bool proc = valid;
-    stop = stop_check(P, valid, Ti, k, lane, proc, n_proc);
-    accumulate(proc, Ti, v, cr, cg, cb, ca);
-    T = T * readlane(incl, 63);
+//
+// MORE (above 256 samples, early termination): classification ends when both rays have a group; a ray
+// that its groups have not stopped takes the chunks that are left, as forward_sweep does.  Classified
+// to the end, an opaque surface made such views slower than with one ray per wave (800x800, 256^3,
+// 512 samples: nearest 289 -> 431 us, 256 now; trilinear 466 -> 568, 402).  Up to 256 samples the ends are
+// at most 5% of the time and the test costs more in sparse scenes.
+struct FwdRay {
+  float T, cr, cg, cb, ca;
+  int n_proc, nk, ng;  // kept samples listed, groups taken
+  bool stop;
+};
+
+__device__ __forceinline__ FwdRay fwd_start(int S, int nk) { return FwdRay{1.f, 0.f, 0.f, 0.f, 0.f, S, nk, 0, false}; }
+
+template <int DT, int INTERP>
+__device__ __forceinline__ void fwd_group(const KParams& P, const Ray& R, int lane, const int* list, FwdRay& f,
+                                          float* ax) {
+  const int idx = (f.ng << 6) + lane;
+  const bool valid = idx < f.nk;
+  const int k = valid ? list[idx] : 0;
+  if (ax && lane == 0) {
+    ax[2 + 2 * f.ng] = f.T;
+    ax[3 + 2 * f.ng] = __int_as_float(k);
   }
-  const float4 c = make_float4(wave_sum(cr), wave_sum(cg), wave_sum(cb), wave_sum(ca));
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+  uint32_t clip;
+  if (valid) eval_kept<DT, INTERP>(P, R, k, v, clip);
+  const float incl = wave_prefix_mul(1.f - v.w);
+  const float Ti = f.T * wave_shift_up(incl, 1.f);
+  bool proc = valid;
+  f.stop = stop_check(P, valid, Ti, k, lane, proc, f.n_proc);
+  accumulate(proc, Ti, v, f.cr, f.cg, f.cb, f.ca);
+  f.T = f.T * readlane(incl, 63);
+  ++f.ng;
+}
+
+__device__ __forceinline__ void fwd_end(int lane, const FwdRay& f, int64_t ray, float* __restrict__ out, float* ax) {
+  const float4 c = make_float4(wave_sum(f.cr), wave_sum(f.cg), wave_sum(f.cb), wave_sum(f.ca));
   if (lane == 0) {
     reinterpret_cast<float4*>(out)[ray] = c;
     if (ax) {
-      ax[0] = __int_as_float(n_proc);
-      ax[1] = __int_as_float(done);
+      ax[0] = __int_as_float(f.n_proc);
+      ax[1] = __int_as_float(f.ng);
     }
   }
 }
 
-template <int DT, int INTERP, int NG>
-__global__ __launch_bounds__(kBlock) void k_render_pair(KParams P, float* __restrict__ out, float* __restrict__ aux) {
+// NR rays whose kept samples of chunks 0 .. c - 1 are listed, their groups in turn.  Two rays in turn read
+// a trilinear sample's eight cells while the neighbour's are still in the cache: 800x800 view, 256^3,
+// 256 samples, every cell occupied 2631 us one ray after the other, 2370 in turn (2156 with one ray per
+// wave); 512 samples, 70% occupied 2083, 1950 (1922); nearest lookup reads too few cells for that (256 samples, 20%
+// occupied: 263 and 294 us).
+template <int DT, int INTERP, bool MORE, int NR>
+__device__ __forceinline__ void fwd_rays(const KParams& P, const Ray (&R)[NR], FwdRay (&f)[NR], const int64_t (&ray)[NR],
+                                         int* const (&list)[NR], int c, int lane, float* __restrict__ out,
+                                         float* __restrict__ aux) {
+  const int S = P.n_samples, nch = (S + 63) >> 6;
+  float* ax[NR];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) ax[r] = aux ? aux + ray[r] * P.aux_stride : nullptr;
+  for (;;) {
+    for (bool any = true; any;) {
+      any = false;
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const int left = f[r].nk - (f[r].ng << 6);
+        if (f[r].stop || left < (MORE && c < nch ? kWave : 1)) continue;
+        fwd_group<DT, INTERP>(P, R[r], lane, list[r], f[r], ax[r]);
+        any = true;
+      }
+    }
+    if (!MORE || c >= nch) break;
+    bool all = true;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      all = all && f[r].stop;
+      if (!f[r].stop) f[r].nk = append_kept<INTERP>(P, R[r], (c << 6) + lane + 1, S, list[r], f[r].nk);
+    }
+    if (all) break;
+    ++c;
+    wave_lds_sync();
+  }
+#pragma unroll
+  for (int r = 0; r < NR; ++r) fwd_end(lane, f[r], ray[r], out, ax[r]);
+}
+
+// Eight waves per SIMD: float32 trilinear takes 67 registers without the bound, and sparse scenes lose 3%.
+template <int DT, int INTERP, int NG, bool MORE>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_render_pair(KParams P, float* __restrict__ out, float* __restrict__ aux) {
   __shared__ int s_list[kWavesPerBlock][2][kWave * NG];
   constexpr int kBatch = NG <= 2 ? NG : 1;  // chunks classified together
   const int lane = threadIdx.x & 63;
@@ -687,9 +739,10 @@ __global__ __launch_bounds__(kBlock) void k_render_pair(KParams P, float* __rest
   setup_ray(P, ray0, RR[0]);
   if (has1) setup_ray(P, ray0 + 1, RR[1]);
   else RR[1] = RR[0];
-  int n0 = 0, n1 = 0;
-  for (int c0 = 0; c0 < NG; c0 += kBatch) {
+  int n0 = 0, n1 = 0, c0 = 0;
+  for (; c0 < NG; c0 += kBatch) {
     if (kBatch < NG && (c0 << 6) >= P.n_samples) break;
+    if (MORE && n0 >= kWave && (n1 >= kWave || !has1)) break;
     bool kp[2][kBatch];
     classify_chunks<INTERP, 2, kBatch>(P, RR, lane, kp, c0);
 #pragma unroll
@@ -705,8 +758,24 @@ __global__ __launch_bounds__(kBlock) void k_render_pair(KParams P, float* __rest
   }
   wave_lds_sync();
   if (n0 > 32 || n1 > 32) {
-    fwd_ray<DT, INTERP, NG>(P, RR[0], ray0, list0, n0, lane, out, aux);
-    if (has1) fwd_ray<DT, INTERP, NG>(P, RR[1], ray0 + 1, list1, n1, lane, out, aux);
+    if constexpr (INTERP == PXL_INTERP_TRILINEAR) {
+      if (has1) {
+        FwdRay f[2] = {fwd_start(P.n_samples, n0), fwd_start(P.n_samples, n1)};
+        const int64_t rays[2] = {ray0, ray0 + 1};
+        int* const lists[2] = {list0, list1};
+        fwd_rays<DT, INTERP, MORE, 2>(P, RR, f, rays, lists, c0, lane, out, aux);
+        return;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      if (r == 1 && !has1) break;
+      const Ray R1[1] = {RR[r]};
+      FwdRay f[1] = {fwd_start(P.n_samples, r ? n1 : n0)};
+      const int64_t rays[1] = {ray0 + r};
+      int* const lists[1] = {r ? list1 : list0};
+      fwd_rays<DT, INTERP, MORE, 1>(P, R1, f, rays, lists, c0, lane, out, aux);
+    }
     return;
   }
   const bool hi = lane >= 32;
@@ -1321,7 +1390,9 @@ int for_ray_pieces(pxl::KParams P, int64_t rays_per_block, F&& fn, const char* w
 // (65537 rays x 192 samples, 110 kept: 318 us against k_render_fwd's 295).  And from as many rays
 // on as fill the chip's 8192 wave slots in pairs: with fewer, half the waves take longer (100^3, 5%
 // occupied, 256 trilinear samples: 4000 rays 8.0 us in pairs and 6.8 one by one, 13000 12.7 and
-// 13.4, 40000 27.8 and 34.1).
+// 13.4, 40000 27.8 and 34.1).  The host does not see how much is occupied: neighbouring rays through
+// the trilinear cells of a large grid that is mostly occupied lose (65536 rays x 512, 256^3: 30%
+// empty 323 us against 253, 95% empty 66 against 81; 640000 rays: 1950 against 1922).
 constexpr int64_t kPairRays = 1 << 14;
 bool use_pairs(const pxl::KParams& P) { return P.occ != nullptr && P.n_samples <= 512 && P.n_rays >= kPairRays; }
 
@@ -1330,10 +1401,11 @@ void launch_fwd(const pxl::KParams& Q, unsigned nb, float* out, float* aux, hipS
   const int S = Q.n_samples;
 #define PXL_LAUNCH_FWD(K) hipLaunchKernelGGL((K), dim3(nb), dim3(pxl::kBlock), 0, s, Q, out, aux)
   if (!use_pairs(Q)) PXL_LAUNCH_FWD((pxl::k_render_fwd<DT, INTERP>));
-  else if (S <= 64) PXL_LAUNCH_FWD((pxl::k_render_pair<DT, INTERP, 1>));
-  else if (S <= 128) PXL_LAUNCH_FWD((pxl::k_render_pair<DT, INTERP, 2>));
-  else if (S <= 256) PXL_LAUNCH_FWD((pxl::k_render_pair<DT, INTERP, 4>));
-  else PXL_LAUNCH_FWD((pxl::k_render_pair<DT, INTERP, 8>));
+  else if (S <= 64) PXL_LAUNCH_FWD((pxl::k_render_pair<DT, INTERP, 1, false>));
+  else if (S <= 128) PXL_LAUNCH_FWD((pxl::k_render_pair<DT, INTERP, 2, false>));
+  else if (S <= 256) PXL_LAUNCH_FWD((pxl::k_render_pair<DT, INTERP, 4, false>));
+  else if (Q.t_stop > 0.f) PXL_LAUNCH_FWD((pxl::k_render_pair<DT, INTERP, 8, true>));
+  else PXL_LAUNCH_FWD((pxl::k_render_pair<DT, INTERP, 8, false>));
 #undef PXL_LAUNCH_FWD
 }
 

@@ -57,7 +57,7 @@ __host__ __device__ inline int64_t bin_ray_runs(int64_t X, int64_t Y, int64_t Z,
 // Where one wave's next group goes: records from `slot`, runs from region slot run0 + n.
 struct BinCursor {
   uint32_t slot, run0, n;
-  bool sums;  // the nearest scatter goes through the workgroup's cell sums
+  CellSums sums;  // nearest: the workgroup's cell sums (no slots: straight to the gradient)
 };
 
 // One group's kept samples as records slot + rank and runs.  Called by the whole wave.

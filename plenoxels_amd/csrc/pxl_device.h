@@ -728,48 +728,45 @@ __device__ __forceinline__ int merge_nearest_runs(int lane, int ns, uint32_t* s_
 // A workgroup's cell sums (nearest lookup, bundles of neighbouring rays): an open-addressed table
 // of cells in LDS with float64 sums of their four channels (ds_add_f32 takes ~195 clocks per wave
 // instruction on gfx950, ds_add_f64 9 to 41).
-constexpr uint32_t kSumSlots = 512, kSumEmpty = 0xffffffffu, kSumProbes = 8;
+constexpr uint32_t kSumEmpty = 0xffffffffu, kSumProbes = 8;
 
-__device__ __forceinline__ uint32_t* sum_keys() {
-  __shared__ uint32_t s_keys[kSumSlots];
-  return s_keys;
-}
+struct CellSums {
+  uint32_t* keys;
+  double* vals;  // channel ch of slot h: vals[ch * slots + h]
+  uint32_t slots;
+};
 
-__device__ __forceinline__ double* sum_vals() {
-  __shared__ double s_vals[kSumSlots * 4];
-  return s_vals;
-}
-
-// Items 0 .. n-1 (n <= 64, cells in s_cell, which is overwritten) into the table; an item that finds
-// no slot within kProbes goes straight to grad.  Four lanes per item, as flush_cells.
-__device__ __forceinline__ void sum_cells(int lane, int n, float* grad, uint32_t* s_cell, const float* sv) {
-  uint32_t* keys = sum_keys();
-  double* vals = sum_vals();
-  constexpr uint32_t kInTable = 0x80000000u;  // cell indices stay below 2^31
-  if (lane < n) {
+// Items 0 .. n-1 (n <= 64, cells in s_cell, which is overwritten) into the table, a lane per item.  Items
+// without a gradient (empty space, where alpha is clipped) take no slot; one that finds none within
+// kSumProbes goes straight to grad, four lanes per item as in flush_cells.
+__device__ __forceinline__ void sum_cells(const CellSums& t, int lane, int n, float* grad, uint32_t* s_cell,
+                                          const float* sv) {
+  constexpr uint32_t kInTable = 0xffffffffu;  // no cell: indices stay below 2^31
+  const float4 v = lane < n ? reinterpret_cast<const float4*>(sv)[lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+  bool left = v.x != 0.f || v.y != 0.f || v.z != 0.f || v.w != 0.f;
+  if (left) {
     const uint32_t cell = s_cell[lane];
-    uint32_t h = (cell * 2654435761u) >> 23;  // the top nine bits: kSumSlots = 512
+    uint32_t h = __umulhi(cell * 2654435761u, t.slots);
     for (uint32_t p = 0; p < kSumProbes; ++p) {
-      const uint32_t was = atomicCAS(keys + h, kSumEmpty, cell);
+      const uint32_t was = atomicCAS(t.keys + h, kSumEmpty, cell);
       if (was == kSumEmpty || was == cell) {
-        s_cell[lane] = h | kInTable;
+        unsafeAtomicAdd(t.vals + h, (double)v.x);
+        unsafeAtomicAdd(t.vals + t.slots + h, (double)v.y);
+        unsafeAtomicAdd(t.vals + 2u * t.slots + h, (double)v.z);
+        unsafeAtomicAdd(t.vals + 3u * t.slots + h, (double)v.w);
+        left = false;
         break;
       }
-      h = (h + 1u) & (kSumSlots - 1u);
+      h = h + 1u == t.slots ? 0u : h + 1u;
     }
+    if (!left) s_cell[lane] = kInTable;
   }
+  if (__ballot(left) == 0ull) return;
   wave_lds_sync();
-  const int ch = lane & 3;
-  for (int base = 0; base < n; base += kWave / 4) {
-    const int it = base + (lane >> 2);
-    if (it < n) {
-      const float v = sv[4 * it + ch];
-      const uint32_t c = s_cell[it];
-      if (v != 0.f) {
-        if (c & kInTable) unsafeAtomicAdd(vals + (c & ~kInTable) * 4u + ch, (double)v);
-        else atomic_add_f32(grad + (size_t)c * 4u + ch, v);
-      }
-    }
+  for (int it = lane >> 2; it < n; it += kWave / 4) {
+    const uint32_t c = s_cell[it], ch = lane & 3u;
+    const float x = sv[4 * it + (int)ch];
+    if (c != kInTable && x != 0.f) atomic_add_f32(grad + (size_t)c * 4u + ch, x);
   }
 }
 
@@ -789,7 +786,7 @@ template <int INTERP, bool RUNS = false>
 __device__ __forceinline__ void scatter_chunk(const KParams& P, const Ray& R, int lane, int k,
                                               bool keep, uint32_t clip, const float4& gv,
                                               float* grad, uint32_t* s_cell, float4* s_val,
-                                              bool sums = false) {
+                                              const CellSums& sums) {
   constexpr int NI = ScatterItems<INTERP>::kPerSample;
   constexpr int NS = ScatterItems<INTERP>::kStageSamples;
   const uint64_t km = __ballot(keep);
@@ -826,8 +823,8 @@ __device__ __forceinline__ void scatter_chunk(const KParams& P, const Ray& R, in
     }
     bool summed = false;
     if constexpr (RUNS && INTERP == PXL_INTERP_NEAREST) {
-      summed = sums;
-      if (summed) sum_cells(lane, n, grad, s_cell, sv);
+      summed = sums.slots != 0u;
+      if (summed) sum_cells(sums, lane, n, grad, s_cell, sv);
     }
     if (!by_runs && !summed) flush_cells(lane, n, grad, s_cell, sv);
     wave_lds_sync();

@@ -194,12 +194,12 @@ __device__ __forceinline__ void reverse_chunk(const KParams& P, const Ray& R, in
 // Per-wave LDS of the kernels that scatter: the kept-sample list and, once the list has been
 // read into registers, the gradient staging area of scatter_chunk (none with BIN: records go
 // straight to memory).
-template <int INTERP, int LIST, bool BIN = false>
+template <int INTERP, int LIST, bool BIN = false, typename List = int>
 struct WaveLds {
   static constexpr int kItems = BIN ? 0 : ScatterItems<INTERP>::kPerChunk;
   static constexpr int kStage = kItems * 20;
-  static constexpr int kBytes = (LIST * 4 > kStage ? LIST * 4 : kStage);
-  static __device__ __forceinline__ int* list(unsigned char* base) { return reinterpret_cast<int*>(base); }
+  static constexpr int kBytes = (LIST * (int)sizeof(List) > kStage ? LIST * (int)sizeof(List) : kStage);
+  static __device__ __forceinline__ List* list(unsigned char* base) { return reinterpret_cast<List*>(base); }
   static __device__ __forceinline__ uint32_t* cells(unsigned char* base) {
     return reinterpret_cast<uint32_t*>(base);
   }
@@ -250,7 +250,7 @@ __device__ __forceinline__ void reverse_sweep(const KParams& P, const Ray& R, in
 // The cursor of a wave whose first ray is `ray` (local index within the launch) in a region of
 // `rays` rays.
 __device__ __forceinline__ BinCursor bin_cursor(const KParams& P, const Bins& B, uint32_t ray, uint32_t rays) {
-  return BinCursor{ray * (uint32_t)P.n_samples, ray / rays * B.run_cap, 0u, false};
+  return BinCursor{ray * (uint32_t)P.n_samples, ray / rays * B.run_cap, 0u, CellSums{}};
 }
 
 // BIN: the registers of six waves per SIMD, eight with half storage (one or two too many without the
@@ -291,6 +291,13 @@ struct LossParams {
   float* beta;
 };
 
+// The pair's sample lists, k - kListBase: bytes beside the cell sums of up to 256 samples, whose LDS they
+// share (train_pair).
+template <int INTERP, int NG, bool RUN>
+using PairList = typename std::conditional<RUN && INTERP == PXL_INTERP_NEAREST && NG == 4, uint8_t, int>::type;
+template <typename List>
+constexpr int kListBase = sizeof(List) == 1 ? 1 : 0;
+
 // The train step of one ray after classification: its kept samples (list[0..nk)) in groups of
 // 64, loss and its gradient, the reverse sweep and the scatter.  `list` may alias the staging
 // area (s_cell, s_val): it is read completely before the first scatter.
@@ -301,9 +308,9 @@ struct LossParams {
 // (sparse256 spills and takes the flush in none of its stages).  Above 256 samples per ray (three
 // waves per SIMD) it is always there.  For nearest lookup RUN stands for the cell sums of bundles
 // of rays (k_train_pair), again where no occupancy is given.
-template <int DT, int INTERP, int NG, bool BIN, bool RUN>
+template <int DT, int INTERP, int NG, bool BIN, bool RUN, typename List>
 __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP, const Ray& R,
-                                          int64_t ray, const float4& tgt, const int* list, int nk,
+                                          int64_t ray, const float4& tgt, const List* list, int nk,
                                           int lane, uint32_t* s_cell, float4* s_val,
                                           float* __restrict__ out, float* __restrict__ grad,
                                           const Bins& B, BinCursor& cur) {
@@ -328,7 +335,7 @@ __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP
     if (g < ng && !stopped) {
       const int idx = (g << 6) + lane;
       const bool valid = idx < nk;
-      const int k = valid ? list[idx] : 0;
+      const int k = valid ? (int)list[idx] + kListBase<List> : 0;
       if constexpr (BIN) {
         uint32_t open = 0u;
         if (valid) eval_kept<DT, INTERP, true, true>(P, R, k, V[g], open);
@@ -434,18 +441,18 @@ __device__ __forceinline__ Ray select_ray(bool second, const Ray& a, const Ray& 
 
 // Rays ray0 (lanes 0-31, list0[0..n0)) and ray0 + 1 (lanes 32-63, list1[0..n1)), n0, n1 <= 32,
 // one group of each; the steps of train_ray with T = 1 and Qn = 0.
-template <int DT, int INTERP, int NG, bool BIN, bool RUN>
+template <int DT, int INTERP, int NG, bool BIN, bool RUN, typename List>
 __device__ __forceinline__ void train_half_pair(const KParams& P, const LossParams& LP,
                                                 const Ray& R0, const Ray& R1, int64_t ray0,
                                                 bool has1, const float4& tgt0, const float4& tgt1,
-                                                const int* list0, int n0, const int* list1, int n1,
+                                                const List* list0, int n0, const List* list1, int n1,
                                                 int lane, uint32_t* s_cell, float4* s_val,
                                                 float* __restrict__ out, float* __restrict__ grad,
                                                 const Bins& B, BinCursor& cur) {
   const bool hi = lane >= 32;
   const int h = lane & 31;
   const bool valid = h < (hi ? n1 : n0);
-  const int k = valid ? (hi ? list1[h] : list0[h]) : 0;
+  const int k = valid ? (int)(hi ? list1[h] : list0[h]) + kListBase<List> : 0;
   const Ray R = select_ray(hi, R0, R1);
   float4 V = make_float4(0.f, 0.f, 0.f, 0.f);
   uint32_t CL = 0u;
@@ -517,14 +524,16 @@ __device__ __forceinline__ void train_half_pair(const KParams& P, const LossPara
 
 // One wave's pair of rays (ray0 < n_rays); mem: the wave's LDS,
 // [ray 0's list, then the scatter staging area | ray 1's list].
-template <int DT, int INTERP, int NG, bool BIN, bool RUN>
+// start(cur) runs once the wave's rays and targets have been asked for.
+template <int DT, int INTERP, int NG, bool BIN, bool RUN, typename Start>
 __device__ __forceinline__ void train_pair(const KParams& P, const LossParams& LP, int64_t ray0, int lane,
                                            unsigned char* mem, float* __restrict__ out, float* __restrict__ grad,
-                                           const Bins& B, BinCursor& cur) {
-  using L = WaveLds<INTERP, kWave * NG, BIN>;
+                                           const Bins& B, BinCursor& cur, Start&& start) {
+  using List = PairList<INTERP, NG, RUN>;
+  using L = WaveLds<INTERP, kWave * NG, BIN, List>;
   const bool has1 = ray0 + 1 < P.n_rays;
-  int* list0 = L::list(mem);
-  int* list1 = reinterpret_cast<int*>(mem + L::kBytes);
+  List* list0 = L::list(mem);
+  List* list1 = reinterpret_cast<List*>(mem + L::kBytes);
   Ray R0, R1;
   setup_ray(P, ray0, R0);
   if (has1) setup_ray(P, ray0 + 1, R1);
@@ -534,6 +543,7 @@ __device__ __forceinline__ void train_pair(const KParams& P, const LossParams& L
   const float4 tgt1 = !has1 ? tgt0
                     : targets ? reinterpret_cast<const float4*>(targets)[ray0 + 1] : camera_target(P, R1);
   const Ray RR[2] = {R0, R1};
+  start(cur);
   // chunks classified together: all of both rays (one memory round trip), except where nearest
   // lookup has eight, which leaves four waves per SIMD for them (100000 rays x 320 samples: 133 us
   // together, 112 one by one; trilinear, bound by its gathers and scatter, 415 and 449)
@@ -548,8 +558,8 @@ __device__ __forceinline__ void train_pair(const KParams& P, const LossParams& L
       const bool k1 = kp[1][c] & has1;
       const int k = ((c0 + c) << 6) + lane + 1;
       const uint64_t km0 = __ballot(kp[0][c]), km1 = __ballot(k1);
-      if (kp[0][c]) list0[n0 + lane_rank(km0)] = k;
-      if (k1) list1[n1 + lane_rank(km1)] = k;
+      if (kp[0][c]) list0[n0 + lane_rank(km0)] = (List)(k - kListBase<List>);
+      if (k1) list1[n1 + lane_rank(km1)] = (List)(k - kListBase<List>);
       n0 += __popcll(km0);
       n1 += __popcll(km1);
     }
@@ -593,39 +603,61 @@ __device__ __forceinline__ bool is_bundle(const KParams& P) {
 
 // Nearest lookup of a dense grid (RUN) adds ~140 runs of samples per ray; where a workgroup's
 // eight rays are neighbours (whole images, even spreads) they reach the same cells, so their sums
-// are formed in LDS first and added once: 128^3, one 800x800 view x 256 samples: 3.76 -> 1.54
-// ms.  Other workgroups add their runs themselves, at the speed they had (100000 random rays of 30
-// views x 256 samples, 128^3: 443 and 444 us).
+// are formed in LDS first and added once: 128^3, one 800x800 view x 256 samples, the step 3.45 ms
+// without the sums, 1.45 with them.  Other workgroups add their runs themselves, within 1% of the speed of a
+// kernel without the table (100000 random rays x 256 samples, 128^3: 500 and 500 us; 95% of the
+// cells empty 152 and 154): above 128 samples byte lists and 468 slots leave room for as many
+// waves as without it, seven per SIMD; up to 128, where more slots are worth as much, 512 and six
+// instead of eight.  Where a bundle adds little -- empty space, early termination -- meeting twice and
+// looking the slots over costs 5 to 20% of the step (400x400 view x 256, 128^3, 95% empty: 176 us
+// without the sums, 196 with them; opaque 120 and 131).
 template <int DT, int INTERP, int NG, bool BIN, bool RUN>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 && DT != PXL_DTYPE_F16 && !RUN ? 5 : 1))) void k_train_pair(KParams P, LossParams LP,
                                                         float* __restrict__ out,
                                                         float* __restrict__ grad, Bins B) {
   // per wave: [ray 0's list, then the scatter staging area | ray 1's list]
-  using L = WaveLds<INTERP, kWave * NG, BIN>;
-  constexpr int kList1 = kWave * NG * 4;
+  using L = WaveLds<INTERP, kWave * NG, BIN, PairList<INTERP, NG, RUN>>;
+  constexpr int kList1 = kWave * NG * sizeof(PairList<INTERP, NG, RUN>);
   __shared__ __align__(16) unsigned char s_mem[kWavesPerBlock][L::kBytes + kList1];
-  // nearest, RUN: the workgroup's cell sums, used when its rays are neighbours
-  constexpr bool kSums = RUN && INTERP == PXL_INTERP_NEAREST;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t ray0 = P.ray_offset + 2 * ((int64_t)blockIdx.x * kWavesPerBlock + wave);
   BinCursor cur{};
-  if constexpr (kSums) {
-    cur.sums = is_bundle(P);  // the same for every wave
-    if (cur.sums) {
-      for (uint32_t i = threadIdx.x; i < kSumSlots; i += kBlock) sum_keys()[i] = kSumEmpty;
-      for (uint32_t i = threadIdx.x; i < kSumSlots * 4; i += kBlock) sum_vals()[i] = 0.0;
+  if constexpr (RUN && INTERP == PXL_INTERP_NEAREST) {
+    // the workgroup's cell sums, used when its rays are neighbours
+    constexpr uint32_t kSlots = NG == 4 ? 468 : 512;
+    __shared__ uint32_t s_keys[kSlots];
+    __shared__ __align__(16) double s_sums[kSlots * 4];
+    auto start = [&](BinCursor& c) {
+      if (!is_bundle(P)) return;  // the same for every wave
+      c.sums = CellSums{s_keys, s_sums, kSlots};
+      for (uint32_t i = threadIdx.x; i < kSlots; i += kBlock) s_keys[i] = kSumEmpty;
+      for (uint32_t i = threadIdx.x; i < kSlots * 2; i += kBlock)
+        reinterpret_cast<double2*>(s_sums)[i] = make_double2(0.0, 0.0);
       __syncthreads();
-    }
-  }
-  if (ray0 < P.n_rays) train_pair<DT, INTERP, NG, BIN, RUN>(P, LP, ray0, lane, s_mem[wave], out, grad, B, cur);
-  if constexpr (kSums) {
-    if (!cur.sums) return;
+    };
+    if (ray0 < P.n_rays) train_pair<DT, INTERP, NG, BIN, RUN>(P, LP, ray0, lane, s_mem[wave], out, grad, B, cur, start);
+    else start(cur);
+    if (cur.sums.slots == 0u) return;
     __syncthreads();  // no wave has left: the decision is the workgroup's
-    for (uint32_t i = threadIdx.x; i < kSumSlots * 4; i += kBlock) {
-      const float v = (float)sum_vals()[i];
-      if (v != 0.f) atomic_add_f32(grad + (size_t)sum_keys()[i >> 2] * 4u + (i & 3u), v);
+    // the slots in use, 64 looked at and then 16 added at a time, four lanes per cell: one request each
+    uint32_t* used = L::cells(s_mem[wave]);
+    for (uint32_t i0 = wave * kWave; i0 < kSlots; i0 += kBlock) {
+      const uint32_t i = i0 + lane, key = i < kSlots ? s_keys[i] : kSumEmpty;
+      const uint64_t m = __ballot(key != kSumEmpty);
+      if (key != kSumEmpty) used[lane_rank(m)] = i;
+      wave_lds_sync();
+      const int n = __popcll(m);
+      for (int it = lane >> 2; it < n; it += kWave / 4) {
+        const uint32_t slot = used[it], ch = lane & 3u;
+        const float v = (float)s_sums[ch * kSlots + slot];
+        if (v != 0.f) atomic_add_f32(grad + (size_t)s_keys[slot] * 4u + ch, v);
+      }
+      wave_lds_sync();
     }
+  } else {
+    if (ray0 < P.n_rays)
+      train_pair<DT, INTERP, NG, BIN, RUN>(P, LP, ray0, lane, s_mem[wave], out, grad, B, cur, [](BinCursor&) {});
   }
 }
 

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from oracle import plain
-from plenoxels_amd import MarchConfig, train_step
+from plenoxels_amd import MarchConfig, pack_occupancy, train_step
 from util import grad_close, say
 
 pytestmark = pytest.mark.gpu
@@ -17,7 +17,7 @@ DEV = torch.device("cuda:0")
                                          (403, 0.3, "mixed"), (403, 0.0, "same")])
 def test_bundle_gradient(S, R, step, kind):
     """step: cells between neighbouring rays.  delta of half a cell down the long axis: runs, and with
-    S = 256 eight rays reach more than the table's 512 cells."""
+    S = 256 eight rays reach more cells than the table has slots."""
     say("bundles", S, R, step, kind)
     dims, pd = (150, 60, 60), 0.1
     g = torch.Generator().manual_seed(S + R)
@@ -41,3 +41,34 @@ def test_bundle_gradient(S, R, step, kind):
     ok, info = grad_close(grad.cpu(), ref.grad)
     say("  ", info)
     assert ok, info
+
+
+@pytest.mark.parametrize("S", [40, 128, 256])
+@pytest.mark.parametrize("dtype,empty,t_stop", [(torch.float32, 0.95, 0.0), (torch.bfloat16, 0.5, 0.1),
+                                                (torch.float16, 1.0, 0.0)])
+def test_bundle_gradient_in_empty_space(S, dtype, empty, t_stop):
+    """Samples whose cell takes no gradient (alpha below zero) take no slot of the table; rays that stop
+    early leave some waves with few samples; a grid that is all empty leaves nothing to add."""
+    say("bundles in empty space", S, dtype, empty, t_stop)
+    dims, pd, R = (70, 60, 50), 0.1, 331
+    g = torch.Generator().manual_seed(S)
+    grid = torch.rand(*dims, 4, generator=g) * 1.2 - 0.1
+    grid[..., 3] = torch.where(torch.rand(dims, generator=g) < empty, -0.1, grid[..., 3].abs() * 0.5)
+    grid = grid.to(dtype).float()
+    o = torch.tensor([[-0.5, 2.0, 2.0]]) + torch.arange(R).unsqueeze(1) * torch.tensor([[0.0, 0.01, 0.03]]) % 2.0
+    d = torch.nn.functional.normalize(torch.tensor([[1.0, 0.03, 0.11]]), dim=1).expand(R, 3).contiguous()
+    tgt = torch.rand(R, 4, generator=g)
+    cfg = MarchConfig(S, pd * 0.4, (0.0, 0.0, 0.0), pd, "nearest", 0.0, t_stop)
+    grad = torch.zeros(*dims, 4, device=DEV)
+    train_step(grid.to(dtype).to(DEV), grad, cfg=cfg, origins=o.contiguous().to(DEV), dirs=d.to(DEV), targets=tgt.to(DEV))
+    if empty == 1.0:
+        assert grad.abs().max() == 0
+        return
+    # with an occupancy of ones the samples go straight to the gradient: the same terms in another order
+    want = torch.zeros(*dims, 4, device=DEV)
+    ones = pack_occupancy(torch.ones(dims, dtype=torch.bool, device=DEV))
+    train_step(grid.to(dtype).to(DEV), want, cfg=cfg, origins=o.contiguous().to(DEV), dirs=d.to(DEV), targets=tgt.to(DEV),
+               occupancy=ones)
+    ok, info = grad_close(grad.cpu(), want.cpu())
+    say("  ", info)
+    assert ok and want.abs().max() > 0, info

@@ -280,6 +280,77 @@ def test_scatter_work_bytes_stay_within_one_launch():
     assert q((1 << 24) + 1) == q((1 << 24) + 2)
 
 
+def test_work_calls_validate_as_the_plain_ones():
+    L = _lib.lib()
+    g, m, r = _valid()
+    m.interp = _lib.INTERP_TRILINEAR
+    p = ctypes.c_void_p(0x1000)
+    loss = _lib.Loss()
+    loss.grad_scale, loss.targets = 1.0, 0x6000
+    step = lambda G, M, R, ls, grad: L.pxl_train_step_work(  # noqa: E731
+        G, M, R, ls, None, grad, p, 1 << 20, None)
+    bwd = lambda G, M, R, go, aux, grad: L.pxl_render_bwd_work(  # noqa: E731
+        G, M, R, go, aux, grad, p, 1 << 20, None)
+    G, M, R, ls = (ctypes.byref(x) for x in (g, m, r, loss))
+    assert step(G, M, R, ls, p) == _lib.PXL_OK and bwd(G, M, R, None, None, None) == _lib.PXL_OK  # no rays
+    assert step(None, M, R, ls, p) == step(G, None, R, ls, p) == step(G, M, None, ls, p) == _lib.PXL_E_INVALID
+    assert step(G, M, R, None, p) == step(G, M, R, ls, None) == _lib.PXL_E_INVALID
+    assert bwd(None, M, R, p, p, p) == bwd(G, None, R, p, p, p) == bwd(G, M, None, p, p, p) == _lib.PXL_E_INVALID
+    r.n_rays = 4
+    assert bwd(G, M, R, None, p, p) == bwd(G, M, R, p, None, p) == bwd(G, M, R, p, p, None) == _lib.PXL_E_INVALID
+    r.n_rays = -1
+    assert step(G, M, R, ls, p) == bwd(G, M, R, p, p, p) == _lib.PXL_E_INVALID
+    r.n_rays, m.n_samples = 4, _lib.TRAIN_MAX_SAMPLES + 1
+    assert step(G, M, R, ls, p) == _lib.PXL_E_INVALID and str(_lib.TRAIN_MAX_SAMPLES) in _lib.last_error()
+
+
+def test_scatter_work_bytes_rule_on_the_host():
+    """No buffer for nearest lookup, no samples and no rays, errors as the other entry points report them."""
+    L = _lib.lib()
+    g, m, _ = _valid()
+    q = lambda n: L.pxl_scatter_work_bytes(ctypes.byref(g), ctypes.byref(m), n)  # noqa: E731
+    assert q(1 << 24) == 0  # nearest
+    m.interp = _lib.INTERP_TRILINEAR
+    assert q(0) == 0 and q(1) == 0 and q(1 << 20) > 0 and q(-1) == _lib.PXL_E_INVALID
+    g.occupancy = 0x7000
+    assert q(1 << 15) == 0 and q(1 << 24) > 0
+    m.n_samples = 0
+    assert q(1 << 24) == 0
+    m.n_samples, m.pd = 16, 0.0
+    assert q(1 << 24) == _lib.PXL_E_INVALID
+    assert L.pxl_scatter_work_bytes(None, ctypes.byref(m), 5) == _lib.PXL_E_INVALID
+    m.pd, g.dims[1] = 0.2, 0
+    assert q(1 << 24) == _lib.PXL_E_INVALID
+
+
+def test_step_tail_validation():
+    """pxl_loss_terms, pxl_tv_grad, pxl_adam_pooled_step, pxl_alpha_occupancy_tv."""
+    L = _lib.lib()
+    p = lambda a: ctypes.c_void_p(a)  # noqa: E731
+    a, b, c, d, e = (p(0x1000 * i) for i in range(1, 6))
+    terms = lambda sq, n, out, work: L.pxl_loss_terms(sq, None, None, n, 1.0, 0.0, 0.0, 0.0, 1.0, out, work, None)  # noqa: E731
+    assert L.pxl_loss_terms_work_bytes() % 16 == 0 and L.pxl_loss_terms_work_bytes() > 0
+    assert terms(a, -1, b, c) == terms(None, 5, b, c) == terms(a, 5, None, c) == terms(a, 5, b, None) == _lib.PXL_E_INVALID
+    assert terms(a, 5, b, p(0x3008)) == _lib.PXL_E_INVALID and "aligned" in _lib.last_error()
+    tv = lambda grid, dims, s, w, grad: L.pxl_tv_grad(grid, *dims, s, w, grad, None)  # noqa: E731
+    ok = (4, 4, 4)
+    assert tv(None, ok, b, c, d) == tv(a, ok, None, c, d) == tv(a, ok, b, None, d) == tv(a, ok, b, c, None) == _lib.PXL_E_INVALID
+    assert tv(p(0x1004), ok, b, c, d) == tv(a, ok, b, c, p(0x4008)) == tv(a, (4, 0, 4), b, c, d) == _lib.PXL_E_INVALID
+    assert tv(a, (2048, 2048, 2048), b, c, d) == _lib.PXL_E_SIZE
+
+    def adam(param=a, go=b, m=c, v=d, gabs=None, dims=ok, k=3, s=1, step=1, half=None, dt=0, ws=e):
+        return L.pxl_adam_pooled_step(param, go, m, v, gabs, *dims, k, s, 1e-2, 0.9, 0.999, 1e-8, step, half, dt, ws, None)
+    for bad in (dict(param=None), dict(go=None), dict(m=None), dict(v=None), dict(ws=None), dict(k=0), dict(k=5), dict(s=0),
+                dict(step=0), dict(dims=(4, 4, 0)), dict(param=p(0x1004)), dict(go=p(0x2008)), dict(gabs=p(0x6004)),
+                dict(ws=p(0x5004)), dict(half=p(0x6004), dt=_lib.DTYPE_BF16), dict(half=p(0x6000), dt=_lib.DTYPE_F32)):
+        assert adam(**bad) == _lib.PXL_E_INVALID, bad
+    g, _, _ = _valid()
+    occ = lambda G, bits, s: L.pxl_alpha_occupancy_tv(G, 1, bits, s, None)  # noqa: E731
+    assert occ(None, a, b) == occ(ctypes.byref(g), None, b) == occ(ctypes.byref(g), a, None) == _lib.PXL_E_INVALID
+    g.dtype = _lib.DTYPE_BF16
+    assert occ(ctypes.byref(g), a, b) == _lib.PXL_E_DTYPE
+
+
 def test_scaled_sum_validation():
     L = _lib.lib()
     assert L.pxl_scaled_sum_work_bytes() == 1024

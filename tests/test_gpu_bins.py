@@ -85,6 +85,47 @@ def test_binned_train_step_equals_direct(dims, R, S, dtype, occupied, t_stop):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dims,R,S,far", [
+    ((90, 97, 101), 5000, 200, False),     # 2028 tiles: two workgroups of tile ranges, the second a part of one
+    ((129, 136, 130), 60000, 200, True),   # 4913 tiles, items of 512 runs, tiles of more than one item
+    ((210, 201, 216), 60000, 200, False),  # 18954 tiles, most of them reached: more items than workgroups
+])
+def test_binned_train_step_of_many_tiles(dims, R, S, far):
+    """Tile counts that take several workgroups for their ranges, whose workgroups may come in any order,
+    and either number of runs per item; more items than the tile sums have workgroups.  far: a third of
+    the rays cross at one place, whose tiles get thousands of runs."""
+    say("bins, many tiles", dims, R, S, far)
+    tiles = 1
+    for n in dims:
+        tiles *= (n + 7) // 8
+    grid, o, d, gmin, pd, delta, tgt = _scene(dims, R, S, 13)
+    if far:  # through the grid's middle
+        mid = torch.tensor(gmin) + torch.tensor(dims) * (pd / 2)
+        o[::3] = mid + 0.2 * torch.rand(o[::3].shape, generator=torch.Generator().manual_seed(1)) - d[::3] * (delta * S / 2)
+    grid, o, d, tgt = (t.to(DEV) for t in (grid, o, d, tgt))
+    cfg = MarchConfig(S, delta, gmin, pd, "trilinear")
+    g, m = _grid_struct(grid, None), cfg.to_struct()
+    n = _lib.lib().pxl_scatter_work_bytes(ctypes.byref(g), ctypes.byref(m), R)
+    assert n > 0  # the rule takes this batch
+    work = torch.full((n,), 0xA5, dtype=torch.uint8, device=DEV)
+    direct, binned = (_train(grid, o, d, tgt, cfg, None, w) for w in (None, work))
+    for a, b in zip(binned[:3], direct[:3]):
+        assert torch.equal(a, b)
+    # where a third of the rays meet, a cell sums ~10^5 FP32 terms directly: sqrt(10^5) * 2^-24 = 2e-5
+    ok, info = grad_close(binned[3], direct[3], rel=4e-5 if far else 1e-5)
+    # the buffer starts with the items and runs it was left with, then the runs of each tile
+    head = work[(-work.data_ptr()) % 256:][:16 + 4 * tiles].view(torch.int32)
+    items, runs, per_tile = int(head[0]), int(head[1]), head[4:]
+    say("  ", info, "tiles", tiles, "items", items, "runs", runs)
+    assert ok, info
+    per_item = 512 if tiles >= 4096 else 96
+    assert runs == int(per_tile.sum()) and items == int(((per_tile + per_item - 1) // per_item).sum())
+    assert tiles > 1024 and tiles % 1024 != 0
+    assert not far or int(per_tile.max()) > per_item
+    assert dims[0] != 210 or items > 16384
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dims,R,S,dtype", [
     ((9, 17, 5), 130, 40, torch.float32),        # two rays share a group of 64 lanes
     ((24, 24, 24), 501, 128, torch.bfloat16),
@@ -124,6 +165,9 @@ def test_render_rays_backward_above_the_bin_threshold(S, interp):
     up = torch.rand(R, 4, generator=torch.Generator().manual_seed(6)) - 0.5
     up[::7] = 0
     leaf = grid.to(DEV).requires_grad_(True)
+    g, m = _grid_struct(leaf.detach(), None), MarchConfig(S, delta, gmin, pd, interp).to_struct()
+    takes_bins = _lib.lib().pxl_scatter_work_bytes(ctypes.byref(g), ctypes.byref(m), R) > 0
+    assert takes_bins == (interp == "trilinear")
     out = render_rays(leaf, o.to(DEV), d.to(DEV), num_samples=S, delta_step=delta, grid_min=gmin, points_distance=pd,
                       interp=interp)
     out.backward(up.to(DEV))
@@ -228,6 +272,8 @@ def test_binned_train_step_in_a_graph():
     grid, o, d, gmin, pd, delta, tgt = _scene((32, 32, 32), R, S, 9)
     grid, o, d, tgt = (t.to(DEV) for t in (grid, o, d, tgt))
     cfg = MarchConfig(S, delta, gmin, pd, "trilinear")
+    g_, m = _grid_struct(grid, None), cfg.to_struct()
+    assert _lib.lib().pxl_scatter_work_bytes(ctypes.byref(g_), ctypes.byref(m), R) > 0
     grad, eager = torch.zeros_like(grid), torch.zeros_like(grid)
 
     def step(out):

@@ -1,9 +1,9 @@
 // pxl_bins.h -- trilinear gradients through tile bins instead of one memory atomic per corner.
 //
 // Measured (float32, 65537 rays x 192 samples through 160x128x145 cells, ~110 kept each): the
-// backward kernel 1426 us with corner atomics; 361 us writing records, then 32 us sorting the
-// runs and 148 us for the tile sums.  A 512^3 BF16 training step's 2^19 rays: 4671 us before;
-// 1784 + 150 + 818 now.
+// backward kernel 1426 us with corner atomics; 341 us writing records, then 24 us sorting the
+// runs and 127 us for the tile sums.  A 512^3 BF16 training step's 2^19 rays: 4671 us before;
+// 1778 + 145 + 805 now.
 // Float atomics run at the memory side at ~20-26 G requests/s device-wide (one request: a
 // 64-byte segment touched by one wave instruction), and a trilinear sample's eight corners
 // need four to five of them.  Here the kernels that produce gradients write one 32-byte record

@@ -497,8 +497,8 @@ __device__ __forceinline__ float clip_ch(float raw, uint32_t& bits, int bit) {
 // storage: the two z neighbours of a row are one 16-byte load (8-byte aligned), which halves the
 // gather instructions; in a row's last cell the pair starts one cell lower, and the ceil, cell 0,
 // is loaded apart (ZPAIR; 128^3 view, 173^2 rays x 200 samples of a dense grid: 58 -> 44 us in BF16).
-// The train kernels that scatter by atomics are bound by those and keep single loads: 283 us
-// against 289 with pairs (201x173x190 BF16, 100003 rays x 300 samples).
+// k_train_pair with atomics (BIN false) keeps single loads: 283 us against 289 with pairs (201x173x190 BF16,
+// 100003 rays x 300 samples).
 template <int DT>
 struct StoredCell {
   typedef uint2 type;

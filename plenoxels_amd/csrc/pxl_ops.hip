@@ -1299,12 +1299,15 @@ void launch_field(const void* grid, int64_t X, int64_t Y, int64_t Z, bool dilate
   const uint32_t slab = pxl::field_slab(X, Y, Z);
   const int64_t units = ((OCC ? (X + 7) / 8 * 8 : X) + slab - 1) / slab * ((Y + 7) / 8 * 2) * ((Z + 63) / 64);
   const dim3 nb((unsigned)std::min<int64_t>(units, pxl::kFieldWorkgroups)), nt(pxl::kFieldThreads);
-  if (dilate)
-    hipLaunchKernelGGL((pxl::k_field<DT, true, OCC, TV>), nb, nt, 0, s, grid, (uint32_t)X, (uint32_t)Y, (uint32_t)Z,
-                       slab, bits, sum);
-  else
-    hipLaunchKernelGGL((pxl::k_field<DT, false, OCC, TV>), nb, nt, 0, s, grid, (uint32_t)X, (uint32_t)Y, (uint32_t)Z,
-                       slab, bits, sum);
+  if constexpr (OCC) {
+    if (dilate) {
+      hipLaunchKernelGGL((pxl::k_field<DT, true, OCC, TV>), nb, nt, 0, s, grid, (uint32_t)X, (uint32_t)Y, (uint32_t)Z,
+                         slab, bits, sum);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((pxl::k_field<DT, false, OCC, TV>), nb, nt, 0, s, grid, (uint32_t)X, (uint32_t)Y, (uint32_t)Z,
+                     slab, bits, sum);
 }
 
 int check_occupancy_out(const pxl_grid* grid, const uint32_t* bits) {

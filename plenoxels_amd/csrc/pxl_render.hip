@@ -1,8 +1,9 @@
 // pxl_render.hip -- fused render / backward / training-step kernels for gfx950 and the
 // C ABI declared in include/pxl.h.
 //
-// Work mapping: one 64-lane wavefront per ray, four rays per 256-thread block (the train step:
-// two rays per wavefront, sharing one group of 64 lanes when each keeps at most 32 samples).
+// Work mapping: one 64-lane wavefront per ray, four rays per 256-thread block (the train step and, with
+// an occupancy, the forward of large batches: two rays per wavefront, sharing one group of 64 lanes when
+// each keeps at most 32 samples).
 //   classify   every sample k = 64c + lane + 1 is placed and tested (in grid, occupied) in
 //              chunks of 64; kept samples are compacted, in order, into a per-wave LDS list
 //   groups     the expensive work (cell loads, clip, interpolation, compositing, scatter)
@@ -14,7 +15,9 @@
 //              q -> alpha_i (c_i, 1) + (1 - alpha_i) q, so dC/dalpha_i = T_i (c_i - S_i)
 //              needs no division by (1 - alpha_i) and stays exact at alpha = 1.
 // Gradients reach the grid through float atomics (global_atomic_add_f32), staged per group
-// in LDS and flushed four lanes per cell.
+// in LDS and flushed four lanes per cell; nearest gradients of neighbouring rays are summed by cell in LDS
+// first (k_train_pair), and large trilinear batches write records that are summed per 8x8x8 tile
+// (pxl_bins.h).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -305,8 +308,10 @@ constexpr int kListBase = sizeof(List) == 1 ? 1 : 0;
 // samples keep five waves per SIMD only without it, so they have it where there is no occupancy
 // -- dense grids, whose rays keep runs of samples in one cell (64^3, 32768 rays x 128 samples into
 // corner blocks: 330 -> 243 us) -- and not for sparse scenes, whose samples rarely share a cell
-// (sparse256 spills and takes the flush in none of its stages).  Above 256 samples per ray (three
-// waves per SIMD) it is always there.  For nearest lookup RUN stands for the cell sums of bundles
+// (sparse256 spills and takes the flush in none of its stages).  A dense batch whose samples step a cell
+// or more takes none either and pays the wave: at most 2.5% (64^3 and 256^3, 32768 rays x 64 to 256
+// samples, one to three cells apart; below a cell 1.4 to 3.5 times faster).  Above 256 samples per ray it is
+// always there (141 registers, three waves per SIMD), sparse scenes included.  For nearest lookup RUN stands for the cell sums of bundles
 // of rays (k_train_pair), again where no occupancy is given.
 template <int DT, int INTERP, int NG, bool BIN, bool RUN, typename List>
 __device__ __forceinline__ void train_ray(const KParams& P, const LossParams& LP, const Ray& R,
@@ -667,8 +672,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 
 // view with 331 nearest samples) and k_train_pair's half-wave group when each ray keeps at most 32 samples, else
 // groups of one ray.  Every value is formed by the operation tree of
 // forward_sweep, so outputs and aux are the same bits.
-// 800x800 view of a 256^3 FP16 grid with ~5% occupancy, 256 trilinear samples: 663 us with
-// one ray per wave, 451 us with two.
+// 800x800 view of a 256^3 FP16 grid with ~5% occupancy, 256 trilinear samples: 634 us with
+// one ray per wave, 427 us with two.
 //
 // MORE (above 256 samples, early termination): classification ends when both rays have a group; a ray
 // that its groups have not stopped takes the chunks that are left, as forward_sweep does.  Classified
@@ -1274,10 +1279,11 @@ constexpr int64_t kMaxRaysPerLaunch = int64_t(1) << 25;
 // and backward).
 constexpr double kBinMinSamples = double(1 << 19), kBinTileSamples = 160.0;
 constexpr double kBinMinSamplesOcc = double(1 << 22), kBinTileSamplesOcc = 512.0;
-// Largest work buffer (a 512^3 training step of 2^19 rays x 512 samples asks for 11.1 GB; in
-// three pieces of a third its tile sums take 2.7 instead of 1.2 ms), and the workgroups of the
-// tile sums, which stride over the items, whose number only the device knows: enough of them for
-// the hardware to balance tiles of different sizes (1536 resident: 0.85 ms there, 8192: 0.82).
+// Largest work buffer (a 512^3 training step of 2^19 rays x 512 samples asks for 11.1 GB; in three
+// pieces of a third its tile sums took 2.7 ms where one piece took 1.2, with the resident workgroups of
+// that build), and the workgroups of the tile sums, which stride over the items, whose number only the
+// device knows: enough of them for the hardware to balance tiles of different sizes (1536 resident:
+// 0.85 ms there, 8192: 0.82).
 constexpr int64_t kBinMaxBytes = int64_t(12) << 30;
 constexpr unsigned kBinWorkgroups = 16384;
 
@@ -1628,7 +1634,9 @@ int pxl_render_bwd_work(const pxl_grid* grid, const pxl_march* march, const pxl_
 
 namespace {
 
-// k_train_pair / k_train_long over one piece of rays.
+// k_train_pair / k_train_long over one piece of rays.  The variants with run flush or cell sums where there
+// is no occupancy, up to 256 samples (both sides: train_ray, k_train_pair); above, nearest lookup has no
+// sums, whose registers made random dense rays slower (100000 x 400 samples, 128^3: 490 -> 509 us).
 template <int DT, int INTERP, bool BIN>
 void launch_train(const pxl::KParams& Q, const pxl::LossParams& LP, unsigned nb, float* out, float* grad,
                          const pxl::Bins& B, hipStream_t s) {

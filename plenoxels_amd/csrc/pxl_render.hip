@@ -675,11 +675,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NG <= 4 
 // 800x800 view of a 256^3 FP16 grid with ~5% occupancy, 256 trilinear samples: 634 us with
 // one ray per wave, 427 us with two.
 //
-// MORE (above 256 samples, early termination): classification ends when both rays have a group; a ray
-// that its groups have not stopped takes the chunks that are left, as forward_sweep does.  Classified
-// to the end, an opaque surface made such views slower than with one ray per wave (800x800, 256^3,
-// 512 samples: nearest 289 -> 431 us, 256 now; trilinear 466 -> 568, 402).  Up to 256 samples the ends are
-// at most 5% of the time and the test costs more in sparse scenes.
+// MORE (above 256 samples, early termination): half way, when both rays have a group, classification ends;
+// a ray that its groups have not stopped takes the chunks that are left, as forward_sweep does.
+// Classified to the end, an opaque surface made such views slower than with one ray per wave (800x800,
+// 256^3, 512 samples: nearest 289 -> 431 us, 308 now; trilinear 467 -> 567, 438).  Sparse views pay 3% for the
+// stop half way (95% empty, 300 samples: nearest 263 and 272 us; with one ray per wave 380); asked after
+// every chunk it is 256 and 402 us against 4 to 8%.  Up to 256 samples the ends are at most 5% of the time.
 struct FwdRay {
   float T, cr, cg, cb, ca;
   int n_proc, nk, ng;  // kept samples listed, groups taken
@@ -761,8 +762,9 @@ __device__ __forceinline__ void fwd_rays(const KParams& P, const Ray (&R)[NR], F
 }
 
 // Eight waves per SIMD: float32 trilinear takes 67 registers without the bound, and sparse scenes lose 3%.
+// MORE has them as well, without the bound's spilled scalars (FP16 trilinear 5% faster).
 template <int DT, int INTERP, int NG, bool MORE>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_render_pair(KParams P, float* __restrict__ out, float* __restrict__ aux) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(MORE ? 6 : 8))) void k_render_pair(KParams P, float* __restrict__ out, float* __restrict__ aux) {
   __shared__ int s_list[kWavesPerBlock][2][kWave * NG];
   constexpr int kBatch = NG <= 2 ? NG : 1;  // chunks classified together
   const int lane = threadIdx.x & 63;
@@ -776,22 +778,31 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
   setup_ray(P, ray0, RR[0]);
   if (has1) setup_ray(P, ray0 + 1, RR[1]);
   else RR[1] = RR[0];
-  int n0 = 0, n1 = 0, c0 = 0;
-  for (; c0 < NG; c0 += kBatch) {
-    if (kBatch < NG && (c0 << 6) >= P.n_samples) break;
-    if (MORE && n0 >= kWave && (n1 >= kWave || !has1)) break;
-    bool kp[2][kBatch];
-    classify_chunks<INTERP, 2, kBatch>(P, RR, lane, kp, c0);
+  int n0 = 0, n1 = 0;
+  auto classify_to = [&](int c0, int end) {
+    for (; c0 < end; c0 += kBatch) {
+      if (kBatch < NG && (c0 << 6) >= P.n_samples) break;
+      bool kp[2][kBatch];
+      classify_chunks<INTERP, 2, kBatch>(P, RR, lane, kp, c0);
 #pragma unroll
-    for (int c = 0; c < kBatch; ++c) {
-      const bool k1 = kp[1][c] & has1;
-      const int k = ((c0 + c) << 6) + lane + 1;
-      const uint64_t km0 = __ballot(kp[0][c]), km1 = __ballot(k1);
-      if (kp[0][c]) list0[n0 + lane_rank(km0)] = k;
-      if (k1) list1[n1 + lane_rank(km1)] = k;
-      n0 += __popcll(km0);
-      n1 += __popcll(km1);
+      for (int c = 0; c < kBatch; ++c) {
+        const bool k1 = kp[1][c] & has1;
+        const int k = ((c0 + c) << 6) + lane + 1;
+        const uint64_t km0 = __ballot(kp[0][c]), km1 = __ballot(k1);
+        if (kp[0][c]) list0[n0 + lane_rank(km0)] = k;
+        if (k1) list1[n1 + lane_rank(km1)] = k;
+        n0 += __popcll(km0);
+        n1 += __popcll(km1);
+      }
     }
+  };
+  int listed = NG;  // chunks
+  if constexpr (MORE) {
+    classify_to(0, NG / 2);
+    if (n0 >= kWave && (n1 >= kWave || !has1)) listed = NG / 2;
+    else classify_to(NG / 2, NG);
+  } else {
+    classify_to(0, NG);
   }
   wave_lds_sync();
   if (n0 > 32 || n1 > 32) {
@@ -800,7 +811,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
         FwdRay f[2] = {fwd_start(P.n_samples, n0), fwd_start(P.n_samples, n1)};
         const int64_t rays[2] = {ray0, ray0 + 1};
         int* const lists[2] = {list0, list1};
-        fwd_rays<DT, INTERP, MORE, 2>(P, RR, f, rays, lists, c0, lane, out, aux);
+        fwd_rays<DT, INTERP, MORE, 2>(P, RR, f, rays, lists, listed, lane, out, aux);
         return;
       }
     }
@@ -811,7 +822,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
       FwdRay f[1] = {fwd_start(P.n_samples, r ? n1 : n0)};
       const int64_t rays[1] = {ray0 + r};
       int* const lists[1] = {r ? list1 : list0};
-      fwd_rays<DT, INTERP, MORE, 1>(P, R1, f, rays, lists, c0, lane, out, aux);
+      fwd_rays<DT, INTERP, MORE, 1>(P, R1, f, rays, lists, listed, lane, out, aux);
     }
     return;
   }

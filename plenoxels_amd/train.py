@@ -140,6 +140,10 @@ class Trainer:
             self._grad_zero = False
         return self._grad
 
+    @grad.setter
+    def grad(self, value):
+        self._grad, self._pooled_grad, self._grad_zero = value, None, False
+
     def _uniforms(self, i):
         if self.uniforms_fn is not None:
             return self.uniforms_fn(i).to(self.dev).float()

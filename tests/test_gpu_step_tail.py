@@ -51,6 +51,9 @@ def test_trainer_grad_after_a_pooled_step(interp, step):
     a.step(step)
     assert a.grad.abs().max() > 0 and torch.equal(a.grad.abs(), a.grad_abs)
     assert a.grad is a.grad
+    buffer = torch.ones_like(a.grad)
+    a.grad = buffer  # another buffer may take its place, whatever it holds
+    assert a.grad is buffer
     # reading it changes nothing that follows
     b.step(step)
     for _ in range(2):
